@@ -204,8 +204,8 @@ __device__ __forceinline__ void store_nodal(WL &W, int el, int a, double2 xy, do
   *reinterpret_cast<double2 *>(&W.nodal[el][4 * a + 2]) = uv;
 }
 
-// Geometry and stress at quadrature point q of element `el` (lane (el, q)).
-template <int P, typename T, typename WL>
+// Geometry and stress at quadrature point q of element `el` (lane (el, q)). COLS: J^-1 is stored by columns.
+template <int P, typename T, bool COLS = false, typename WL>
 __device__ __forceinline__ void stage_geometry(WL &W, const Basis1D &B, const Material &m, int el, int q) {
   constexpr int NP = Ord<P>::NP;
   const int qx = q % NP, qy = q / NP;
@@ -252,8 +252,8 @@ __device__ __forceinline__ void stage_geometry(WL &W, const Basis1D &B, const Ma
   const double sxy = mu * (G01 + G10);
   const double s = (B.w[qx] * B.w[qy]) * detJ * m.t;
   double *g = &W.geo[el][8 * q];
-  *reinterpret_cast<double2 *>(g + 0) = make_double2(i00, i01);
-  *reinterpret_cast<double2 *>(g + 2) = make_double2(i10, i11);
+  *reinterpret_cast<double2 *>(g + 0) = make_double2(i00, COLS ? i10 : i01);
+  *reinterpret_cast<double2 *>(g + 2) = make_double2(COLS ? i01 : i10, i11);
   *reinterpret_cast<double2 *>(g + 4) = make_double2(s, s * sxx);
   *reinterpret_cast<double2 *>(g + 6) = make_double2(s * syy, s * sxy);
 }
@@ -512,90 +512,103 @@ __global__ __launch_bounds__(WAVES * 64) void element_kernel(const ElemArgs args
 }
 
 // ---- element-once assembly of a plan with split tables, orders 3-4 -----------------------------------
-// K_e is formed in tiles of 4 x 4 nodes, one tile per lane, upper tiles only (K_e is symmetric): for G =
-// ceil(N / 4) node groups, tile t of an element covers rows 4I..4I+3 and columns 4J..4J+3, I <= J, in the
-// order (0,0), (0,1), .., (0,G-1), (1,1), ... Per quadrature point each lane (el, a) publishes node a's
-// physical gradient n_a and its weighted copy s_q n_a (adding node a's residual terms), and each tile lane
-// reads the weighted gradients of its 4 rows and the gradients of its 4 columns and adds the Gram sums of
-// its 16 blocks: 64 FMAs for 8 LDS reads.
-// Calls f(std::integral_constant<int, i>) for i = 0 .. n-1, each call a separate instantiation.
-template <typename F, int... Is>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, Is...>) {
-  (f(std::integral_constant<int, Is>{}), ...);
-}
-template <int n, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-  static_for_impl(f, std::make_integer_sequence<int, n>{});
-}
-
+// The Gram sums of an element are one product C = A B on the matrix cores, over the quadrature points q:
+//   A[(a, alpha)][q] = s_q dN_a/dx_alpha(q),  B[q][(b, beta)] = dN_b/dx_beta(q),  C = S_alpha,beta(a, b),
+// in 16 x 16 tiles of 8 x 8 nodes, upper tiles only (K_e is symmetric), four points per step
+// (v_mfma_f64_16x16x4_f64 / v_mfma_f32_16x16x4_f32; both add the four products as an ascending chain of
+// fused multiply-adds, so the sums are those of a loop over the points). Lane l supplies row / column l % 16 of
+// point l / 16 of a step: A and B take the same node and component, so a lane forms one gradient component
+// per 8 nodes and scales it. Order 3 is 2 groups of 8 nodes; order 4 is 3 groups and node 24, whose 25 sums
+// are formed on the vector ALU by lane (el, a) beside the residual (a fourth group would be 7/8 padding).
 template <int P>
-struct TileMap {
-  static constexpr int N = Ord<P>::N;
-  static constexpr int G = (N + 3) / 4;
-  static constexpr int T = G * (G + 1) / 2;
-  static_assert(Ord<P>::EPW * T <= 64, "the tiles of a wavefront's elements exceed its lanes");
+struct GramTiles {
+  static constexpr int N = Ord<P>::N, Q = Ord<P>::Q;
+  static constexpr int G8 = N / 8;                // groups of 8 nodes
+  static constexpr int REST = N - 8 * G8;         // nodes past them (order 4: 1)
+  static constexpr int T = G8 * (G8 + 1) / 2;     // upper tiles (I, J), I <= J, in the order (0,0), (0,1), ..
+  static constexpr int STEPS = (Q + 3) / 4;
+  static_assert(P >= 3 && REST <= 1, "orders 3-4");
 };
 
-// The emission's store instructions: group R of 4 rows takes iters(R) instructions (16 blocks each over
-// the wavefront's elements), issued in chunks of CHK whose destination codes are loaded one chunk ahead
-// (order 3: 16 instructions per group in two chunks, so the codes fit the registers beside the Gram tiles).
-template <int P>
-struct EmitPlan {
-  static constexpr int N = Ord<P>::N, EPW = Ord<P>::EPW, G = TileMap<P>::G;
-  static constexpr int CHK = P == 3 ? 8 : 16;
-  static constexpr int iters(int R) { return (EPW * (N - 4 * R < 4 ? N - 4 * R : 4) * N + 15) / 16; }
-  static constexpr int chunks(int R) { return (iters(R) + CHK - 1) / CHK; }
-  static constexpr int steps() {
-    int t = 0;
-    for (int R = 0; R < G; R++) t += chunks(R);
-    return t;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+// Half a block (16 bytes) of caller memory, which need only be aligned as a double.
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// The value of lane l ^ 1 (a quad permutation), 32 bits at a time.
+template <typename T>
+__device__ __forceinline__ T lane_xor1(T v) {
+  constexpr int W = int(sizeof(T) / 4);
+  int w[W];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (int i = 0; i < W; i++) w[i] = __builtin_amdgcn_mov_dpp(w[i], 0xB1, 0xf, 0xf, true);
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+
+// How the two product instructions spread a tile over the wavefront. Lane l, j = l % 16, g = l / 16:
+// node(j) and component j & 1 is what lane l supplies for row and column j; pair(C, p) gives the lane's sums
+// (S_0,beta, S_1,beta) of row node row(g) + 4p, p = 0, 1, column node node(j) and beta = j & 1.
+template <typename T>
+struct TileLanes;
+template <>
+struct TileLanes<double> {
+  // C[4 r + g][j] in register r: the row components alternate with g, so registers 2p and 2p+1 trade
+  // 16-lane rows (v_permlane16_swap).
+  using V4 = doublex4;
+  static __device__ __forceinline__ int node(int j) { return j >> 1; }
+  static __device__ __forceinline__ int row(int g) { return (g >> 1) + 2 * (g & 1); }
+  static __device__ __forceinline__ V4 mfma(double a, double b, V4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static constexpr int group(int k) {
-    for (int R = 0; R < G; R++) {
-      if (k < chunks(R)) return R;
-      k -= chunks(R);
-    }
-    return G - 1;
+  static __device__ __forceinline__ void pair(const V4 &c, int p, double &s0, double &s1) {
+    const double even = c[2 * p], odd = c[2 * p + 1];
+    const uint2 x = __builtin_bit_cast(uint2, even), y = __builtin_bit_cast(uint2, odd);
+    const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+    s0 = __builtin_bit_cast(double, make_uint2(lo[0], hi[0]));
+    s1 = __builtin_bit_cast(double, make_uint2(lo[1], hi[1]));
   }
-  static constexpr int chunk(int k) {
-    for (int R = 0; R < G; R++) {
-      if (k < chunks(R)) return k;
-      k -= chunks(R);
-    }
-    return 0;
+};
+template <>
+struct TileLanes<float> {
+  // C[4 g + r][j] in register r.
+  using V4 = floatx4;
+  static __device__ __forceinline__ int node(int j) { return 4 * ((j >> 1) & 1) + (j >> 2); }
+  static __device__ __forceinline__ int row(int g) { return g; }
+  static __device__ __forceinline__ V4 mfma(float a, float b, V4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void pair(const V4 &c, int p, float &s0, float &s1) {
+    s0 = c[2 * p];
+    s1 = c[2 * p + 1];
   }
 };
 
+// k s + mu o, the block component from its two sums. FP32: the product fused into the addition is the own one
+// (`own`) or the other, a fixed rule per component and node pair.
+__device__ __forceinline__ double block_sum(double k, double s, double mu, double o, bool) { return fma(k, s, mu * o); }
+__device__ __forceinline__ float block_sum(float k, float s, float mu, float o, bool own) {
+  return fmaf(own ? k : mu, own ? s : o, (own ? mu : k) * (own ? o : s));
+}
+
+// Per-wave LDS: the gathered nodes, then the emission staging of a group of 8 rows of K_e (block (i, b) of the
+// group at kidx(i, b): rows padded to an odd number of 32-byte (FP64) or 16-byte blocks, so that neither the
+// direct nor the transposed writes of a tile meet in a bank), and each point's geometry (J^-1 by columns, s,
+// s * sigma).
 template <int P, typename T>
 struct __align__(16) WaveLDSTile {
   using O = Ord<P>;
-  using V2 = typename Vec2<T>::type;
-  static constexpr int PUB_STRIDE = odd_units(O::N, int(sizeof(V2)));
-  // Emission staging of one group of 4 rows: plane 0 holds (K_xx, K_xy) and plane 1 (K_yx, K_yy) of block
-  // (el, row i, column b) at kidx(el, i, b). Column b sits at b + b/4 and elements are an odd number of
-  // 2-vectors apart, so the lanes of one staging write (one per tile: columns 4 apart) hit distinct banks.
-  static constexpr int KROW = O::N + O::N / 4 + 1;
-  static constexpr int KEL = 4 * KROW + 1;
-  union {
-    double nodal[O::EPW][O::NODAL_STRIDE];  // x, y, u, v of each element node
-    V2 pub[2][2][O::EPW][PUB_STRIDE];       // [buffer][n_a, s_q n_a][el][a] at the current point
-    V2 kq[2][O::EPW * KEL];
+  static constexpr int KROW = O::N | 1;
+  struct __align__(16) Block {
+    T k[4];
   };
-  double geo[O::EPW][O::GEO_STRIDE];  // as WaveLDS::geo
-
-  static __device__ __forceinline__ int kidx(int el, int i, int b) { return el * KEL + i * KROW + b + b / 4; }
-  __device__ __forceinline__ void put(int el, int i, int b, T k0, T k1, T k2, T k3) {
-    V2 lo, hi;
-    lo.x = k0;
-    lo.y = k1;
-    hi.x = k2;
-    hi.y = k3;
-    kq[0][kidx(el, i, b)] = lo;
-    kq[1][kidx(el, i, b)] = hi;
-  }
-  __device__ __forceinline__ T get(int el, int i, int b, int c) const {
-    return reinterpret_cast<const T *>(&kq[c >> 1][kidx(el, i, b)])[c & 1];
-  }
+  union {
+    double nodal[O::EPW][O::NODAL_STRIDE];
+    Block k[8 * KROW];
+  };
+  double geo[O::EPW][O::GEO_STRIDE];
 };
 
 // One element-once assembly: a plan's element-once tables and a request's inputs and outputs.
@@ -603,7 +616,8 @@ struct SplitJob {
   const int *conn;   // [E][N]
   const int *code;   // [E][N][N] block codes (SplitHost::code)
   const int *rcode;  // [E][N] residual codes
-  const int *gdst, *gptr, *rdst, *rptr;  // gather lists of the staged blocks and residual entries
+  const int *gline, *gptr, *gsrc;  // gather list of the staged blocks (GatherList)
+  const int *rline, *rptr, *rsrc;  // and of the staged residual entries
   const double *states, *coords;
   double *residual;  // NULL: no residual
   double *values;
@@ -613,207 +627,201 @@ struct SplitJob {
   int accumulate;  // 1: outputs are added to (+=), staging is still written
 };
 
-// Elements first .. first+EPW-1 of `job` (those below job.count) on one wavefront: geometry, Gram tiles,
-// residual and emission. Every lane of the wavefront calls it; it synchronises the wavefront only.
+// Elements first .. first+EPW-1 of `job` (those below job.count) on one wavefront: geometry, residual, Gram
+// tiles and emission. Every lane of the wavefront calls it; it synchronises the wavefront only.
 template <int P, typename T, bool RES, bool ACC = false>
 __device__ __forceinline__ void tiled_wave(WaveLDSTile<P, T> &W, const Basis1D &basis, const double2 *gref,
                                            const SplitJob &job, int64_t first, int lane) {
   using O = Ord<P>;
-  using TM = TileMap<P>;
+  using GT = GramTiles<P>;
+  using L = TileLanes<T>;
   using V2 = typename Vec2<T>::type;
-  constexpr int N = O::N, Q = O::Q, EPW = O::EPW, NT = TM::T;
+  constexpr int N = O::N, Q = O::Q, EPW = O::EPW, G8 = GT::G8, KROW = WaveLDSTile<P, T>::KROW;
   static_assert(Q == N, "lane (el, q) of the geometry stage is lane (el, a)");
   wave_sync();  // a previous call's LDS reads are done before the nodes overwrite them
-  if (first >= job.count) return;  // no element: the emission below assumes at least one
+  if (first >= job.count) return;
+  const T mu = T(job.mat.mu), lam = T(job.mat.lambda), c1 = lam + 2 * mu;
   // node role: lane (el, a)
   const int el = lane / N, a = lane % N;
   const bool nvalid = lane < EPW * N && first + el < job.count;
-  const int elc = el < EPW ? el : EPW - 1;
-  int node = 0;
   if (nvalid) {
-    node = job.conn[(first + el) * N + a];
+    const int node = job.conn[(first + el) * N + a];
     store_nodal(W, el, a, *reinterpret_cast<const double2 *>(job.coords + 2 * int64_t(node)),
                 *reinterpret_cast<const double2 *>(job.states + 2 * int64_t(node)));
   }
   wave_sync();
-  if (nvalid) stage_geometry<P, T>(W, basis, job.mat, el, a);
+  if (nvalid) stage_geometry<P, T, true>(W, basis, job.mat, el, a);
   wave_sync();
-  // tile role: lane (te, t)
-  const int te = lane / NT;
-  const bool tvalid = lane < EPW * NT && first + te < job.count;
-  const int tec = te < EPW ? te : EPW - 1;
-  int I = 0, J = 0;
-  {
-    int r = lane < EPW * NT ? lane % NT : 0;
-    while (r >= TM::G - I) {
-      r -= TM::G - I;
-      I++;
+  T kr[4] = {0, 0, 0, 0};  // order 4: K(a, N - 1)
+  if (RES || GT::REST) {
+    const int elc = el < EPW ? el : EPW - 1;
+    double Rx = 0, Ry = 0;
+    T S[4] = {0, 0, 0, 0};  // [xx, yy, xy, yx] of nodes (a, N - 1)
+#pragma unroll 5
+    for (int q = 0; q < Q; q++) {
+      const double *g = &W.geo[elc][8 * q];
+      const double2 gr = gref[q * N + a];
+      const double2 cx = *reinterpret_cast<const double2 *>(g), cy = *reinterpret_cast<const double2 *>(g + 2);
+      const double2 sc = *reinterpret_cast<const double2 *>(g + 4), sd = *reinterpret_cast<const double2 *>(g + 6);
+      const double nxd = gr.x * cx.x + gr.y * cx.y, nyd = gr.x * cy.x + gr.y * cy.y;
+      if (RES) {
+        Rx += sc.y * nxd + sd.y * nyd;
+        Ry += sd.y * nxd + sd.x * nyd;
+      }
+      if constexpr (GT::REST > 0) {
+        const double2 gn = gref[q * N + N - 1];
+        const T bx = T(gn.x * cx.x + gn.y * cx.y), by = T(gn.x * cy.x + gn.y * cy.y);
+        const T s = T(sc.x), vx = s * T(nxd), vy = s * T(nyd);
+        S[0] = fma(vx, bx, S[0]);
+        S[1] = fma(vy, by, S[1]);
+        S[2] = fma(vx, by, S[2]);
+        S[3] = fma(vy, bx, S[3]);
+      }
     }
-    J = I + r;
+    if (RES && nvalid) {
+      const int rc = job.rcode[(first + el) * N + a];
+      const bool direct = rc < job.numNodes;
+      double *base = direct ? job.residual : job.rstage - 2 * int64_t(job.numNodes);
+      auto *r = reinterpret_cast<FEM_GLOBAL_AS double2u *>(gmem_mut(base + 2 * int64_t(rc)));
+      double2u d = {Rx, Ry};
+      if (ACC && direct) d += *r;
+      *r = d;
+    }
+    if constexpr (GT::REST > 0) {
+      const bool low = a % 4 > (N - 1) % 4;
+      kr[0] = block_sum(c1, S[0], mu, S[1], true);
+      kr[1] = block_sum(lam, S[2], mu, S[3], low);
+      kr[2] = block_sum(lam, S[3], mu, S[2], !low);
+      kr[3] = block_sum(c1, S[1], mu, S[0], false);
+    }
   }
-  int rows[4], cols[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    rows[k] = min(4 * I + k, N - 1);  // past the last node: a real node, not emitted
-    cols[k] = min(4 * J + k, N - 1);
-  }
-  T S[4][4][4];  // [row][col][xx, yy, xy, yx]
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) S[i][j][0] = S[i][j][1] = S[i][j][2] = S[i][j][3] = 0;
-  double Rx = 0, Ry = 0;
+  // tile role
+  const int j = lane & 15, g = lane >> 4, beta = j & 1;
+  const int nb = L::node(j), na = L::row(g);
+  const T kA = beta ? lam : c1, kB = beta ? c1 : lam;
+  const bool low = na % 4 > nb % 4, own0 = !beta || low, own1 = !beta && !low;
+  const int elements = int(min<int64_t>(EPW, job.count - first));
 #pragma unroll 1
-  for (int q = 0; q < Q; q++) {
-    const int buf = q & 1;
-    PointGeo G;
-    load_point<P, T>(W, gref, elc, a < N ? a : 0, q, G);
-    T nx, ny;
-    V2 v;
-    point_terms<T, V2>(G, nx, ny, v, Rx, Ry);
-    if (nvalid) {
-      W.pub[buf][0][el][a].x = nx;
-      W.pub[buf][0][el][a].y = ny;
-      W.pub[buf][1][el][a] = v;
+  for (int e = 0; e < elements; e++) {
+    // Destination codes in emission order, on their way during the products: lane pair (2k, 2k+1) stores block
+    // 32 it + k of a group of 8 rows (row-major), each lane one 16-byte half.
+    constexpr int GB = 8 * N, IT = (GB + 31) / 32;
+    const int *code = job.code + (first + e) * N * N;
+    int at[G8][IT], atr = 0;
+#pragma unroll
+    for (int R = 0; R < G8; R++) {
+#pragma unroll
+      for (int it = 0; it < IT; it++) at[R][it] = code[R * GB + min(32 * it + (lane >> 1), GB - 1)];
     }
-    wave_sync();  // a buffer is rewritten two points after it was read; a wavefront's LDS accesses run in order
-    V2 rw[4], cn[4];
+    if (GT::REST) atr = code[(N - 1) * N + min(lane >> 1, N - 1)];
+    typename L::V4 C[GT::T];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      rw[k] = W.pub[buf][1][tec][rows[k]];
-      cn[k] = W.pub[buf][0][tec][cols[k]];
+    for (int t = 0; t < GT::T; t++) C[t] = typename L::V4{0, 0, 0, 0};
+#pragma unroll
+    for (int st = 0; st < GT::STEPS; st++) {
+      const bool pad = 4 * st + g >= Q;  // past the last point: weight 0
+      const int q = pad ? Q - 1 : 4 * st + g;
+      const double *geo = &W.geo[e][8 * q];
+      const double2 jc = *reinterpret_cast<const double2 *>(geo + 2 * beta);
+      const T s = pad ? T(0) : T(geo[4]);
+      T n[G8], v[G8];
+#pragma unroll
+      for (int k = 0; k < G8; k++) {
+        const double2 gr = gref[q * N + 8 * k + nb];
+        n[k] = T(gr.x * jc.x + gr.y * jc.y);
+        v[k] = s * n[k];
+      }
+#pragma unroll
+      for (int I = 0, t = 0; I < G8; I++)
+#pragma unroll
+        for (int J = I; J < G8; J++, t++) C[t] = L::mfma(v[I], n[J], C[t]);
     }
+    // Sums to block components, in place: C[t][2p], C[t][2p+1] = K_0,beta, K_1,beta of the lane's column.
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int t = 0; t < GT::T; t++) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        S[i][j][0] = fma(rw[i].x, cn[j].x, S[i][j][0]);
-        S[i][j][1] = fma(rw[i].y, cn[j].y, S[i][j][1]);
-        S[i][j][2] = fma(rw[i].x, cn[j].y, S[i][j][2]);
-        S[i][j][3] = fma(rw[i].y, cn[j].x, S[i][j][3]);
+      for (int p = 0; p < 2; p++) {
+        T s0, s1;
+        L::pair(C[t], p, s0, s1);
+        const T o0 = lane_xor1(s0), o1 = lane_xor1(s1);
+        C[t][2 * p] = block_sum(kA, s0, mu, o1, own0);
+        C[t][2 * p + 1] = block_sum(kB, s1, mu, o0, own1);
       }
     }
-  }
-  if (RES && nvalid) {
-    const int rc = job.rcode[(first + el) * N + a];
-    double *r = rc < job.numNodes ? job.residual + 2 * int64_t(rc) : job.rstage + 2 * (int64_t(rc) - job.numNodes);
-    if (ACC && rc < job.numNodes) {
-      Rx += r[0];
-      Ry += r[1];
-    }
-    __builtin_nontemporal_store(Rx, r);
-    __builtin_nontemporal_store(Ry, r + 1);
-  }
-  // The tile's blocks K(a, b), row-major [xx, xy, yx, yy], in place of its Gram sums.
-  {
-    const T mu = T(job.mat.mu), lam = T(job.mat.lambda), c1 = lam + 2 * mu;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const T xx = S[i][j][0], yy = S[i][j][1], xy = S[i][j][2], yx = S[i][j][3];
-        S[i][j][0] = c1 * xx + mu * yy;
-        S[i][j][1] = lam * xy + mu * yx;
-        S[i][j][2] = lam * yx + mu * xy;
-        S[i][j][3] = c1 * yy + mu * xx;
+    auto store_rows = [&](int it, int count, int code) __attribute__((always_inline)) {
+      const int k = 32 * it + (lane >> 1);
+      if (32 * it + 32 <= count || k < count) {
+        const int i = k / N, h = lane & 1;
+        const V2 v = reinterpret_cast<const V2 *>(W.k[i * KROW + k - i * N].k)[h];
+        const bool direct = code < job.numBlocks;
+        double *base = direct ? job.values : job.stage - 4 * int64_t(job.numBlocks);
+        auto *dst = reinterpret_cast<FEM_GLOBAL_AS double2u *>(gmem_mut(base + 4 * int64_t(code) + 2 * h));
+        double2u d = {double(v.x), double(v.y)};
+        if (ACC && direct) d += *dst;
+        *dst = d;
       }
-    }
-  }
-  // Emission, one group of 4 rows at a time: the tiles holding blocks of rows 4R..4R+3 write them to LDS
-  // (tile (R, J) directly; tile (J, R), J < R, transposed: K(b, a) = K(a, b)^T), then each store instruction
-  // covers the four components of 16 consecutive blocks of the group's rows (lanes 4k..4k+3: block k). The
-  // destination codes of the next chunk of stores (EmitPlan) are loaded while the current chunk is stored.
-  // Every code load and store is unconditional, so that the wait for a chunk's codes lets the previous
-  // chunk's stores stay in flight:
-  // lanes past the group's last block (or past the wavefront's last element) repeat the store of that block,
-  // the same value to the same address in the same instruction.
-  using EP = EmitPlan<P>;
-  constexpr int CHK = EP::CHK;
-  const int c = lane & 3;
-  const int lastEl = int(min<int64_t>(EPW, job.count - first)) - 1;
-  // block (e, rem) of store instruction `it` of group R (rem: offset within the element's rows of the group);
-  // dup: the lane repeats another lane's block (past the group's last block or the wavefront's last element)
-  auto locate = [&](int R, int it, int &e, int &rem, bool &dup) __attribute__((always_inline)) {
-    const int groupBlocks = (N - 4 * R < 4 ? N - 4 * R : 4) * N;
-    const int want = 16 * it + (lane >> 2);
-    dup = want > EPW * groupBlocks - 1;
-    rem = min(want, EPW * groupBlocks - 1);
-    e = 0;
+    };
+    auto tile_at = [](int I, int J) { return I * G8 - I * (I - 1) / 2 + J - I; };
 #pragma unroll
-    for (int k = 1; k < EPW; k++) {
-      if (rem >= groupBlocks) {
-        rem -= groupBlocks;
-        e++;
+    for (int R = 0; R < G8; R++) {
+      wave_sync();  // the previous rows' (or the geometry's) LDS reads are done
+#pragma unroll
+      for (int J = 0; J < G8; J++) {
+        const auto &K = C[tile_at(J < R ? J : R, J < R ? R : J)];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+          // Mixed precision takes the lower 4 x 4 corner of a diagonal tile from the upper one, transposed.
+          const bool half = J == R && sizeof(T) == 4;
+          if (J >= R && !(half && p == 1 && nb < 4)) {
+            T *k = W.k[(4 * p + na) * KROW + 8 * J + nb].k;
+            k[beta] = K[2 * p];
+            k[2 + beta] = K[2 * p + 1];
+          }
+          if (J < R || (half && p == 0 && nb >= 4)) {  // K(b, a) = K(a, b)^T
+            T *k = W.k[nb * KROW + 8 * J + 4 * p + na].k;
+            V2 v;
+            v.x = K[2 * p];
+            v.y = K[2 * p + 1];
+            reinterpret_cast<V2 *>(k)[beta] = v;
+          }
+        }
       }
-    }
-    if (e > lastEl) {
-      e = lastEl;
-      rem = groupBlocks - 1;
-      dup = true;
-    }
-  };
-  int cur[CHK], nxt[CHK];
-  // codes of step k: chunk EP::chunk(k) of group EP::group(k)
-  auto load_codes = [&](auto Kc, int (&at)[CHK]) __attribute__((always_inline)) {
-    constexpr int k = decltype(Kc)::value, R = EP::group(k), ch = EP::chunk(k);
+      if (GT::REST && el == e && a / 8 == R) {
+        T *k = W.k[(a - 8 * R) * KROW + N - 1].k;
 #pragma unroll
-    for (int it = 0; it < CHK; it++) {
-      if (ch * CHK + it >= EP::iters(R)) break;
-      int e, rem;
-      bool dup;
-      locate(R, ch * CHK + it, e, rem, dup);
-      at[it] = job.code[((first + e) * N + 4 * R) * N + rem];
-    }
-  };
-  load_codes(std::integral_constant<int, 0>{}, cur);
-  static_for<EP::steps()>([&](auto Kc) __attribute__((always_inline)) {
-    constexpr int k = decltype(Kc)::value, R = EP::group(k), ch = EP::chunk(k);
-    if constexpr (k + 1 < EP::steps()) load_codes(std::integral_constant<int, k + 1>{}, nxt);
-    if constexpr (ch == 0) {
-      wave_sync();  // the previous group's (or the last point's) LDS reads are done
-      if (tvalid && I == R) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            if (4 * I + i < N && 4 * J + j < N) W.put(tec, i, 4 * J + j, S[i][j][0], S[i][j][1], S[i][j][2], S[i][j][3]);
-      } else if (tvalid && J == R) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++)
-            if (4 * J + j < N) W.put(tec, j, 4 * I + i, S[i][j][0], S[i][j][2], S[i][j][1], S[i][j][3]);
+        for (int c = 0; c < 4; c++) k[c] = kr[c];
       }
       wave_sync();
-    }
 #pragma unroll
-    for (int it = 0; it < CHK; it++) {
-      if (ch * CHK + it >= EP::iters(R)) break;
-      int e, rem;
-      bool dup;
-      locate(R, ch * CHK + it, e, rem, dup);
-      const int at = cur[it];
-      const int i = rem / N, b = rem - i * N;
-      double *blkp = at < job.numBlocks ? job.values + 4 * int64_t(at) : job.stage + 4 * (int64_t(at) - job.numBlocks);
-      double val = double(W.get(e, i, b, c));
-      if (!ACC) {
-        __builtin_nontemporal_store(val, blkp + c);
-      } else if (!dup) {
-        // accumulate mode: each block added once (repeating lanes store nothing); staging is written
-        if (at < job.numBlocks) val += blkp[c];
-        __builtin_nontemporal_store(val, blkp + c);
+      for (int it = 0; it < IT; it++) store_rows(it, GB, at[R][it]);
+    }
+    if (GT::REST) {  // the last row: the transposes of the last column
+      wave_sync();
+      if (el == e && a < N) {
+        T *k = W.k[a].k;
+        const bool t = a < N - 1;
+        k[0] = kr[0];
+        k[1] = t ? kr[2] : kr[1];
+        k[2] = t ? kr[1] : kr[2];
+        k[3] = kr[3];
       }
+      wave_sync();
+      store_rows(0, N, atr);
     }
-#pragma unroll
-    for (int it = 0; it < CHK; it++) cur[it] = nxt[it];
-  });
+  }
 }
 
-
-// Two wavefronts per SIMD, which the LDS of two 4-wavefront workgroups per CU allows: without the bound the FP64
-// order-3 kernel takes 259 registers and runs one wavefront per SIMD (order 3 FP64: 1.40 against 1.50 ms).
+// What bounds it (annulus 200 x 1250 order 4, FP64, 1.66 ms of the assembly's 2.17): the 5.4 GB of stores. Without
+// its stores the kernel takes 0.87 ms, with every store at consecutive addresses 1.35 ms; with 1, 2 or 4 wavefronts
+// per SIMD and with the products or the geometry left out the time is the same. Hence the emission in row order:
+// a row of K_e is a few runs of consecutive blocks. Stored straight from the tiles (8 x 8 blocks, lower tiles
+// column by column) the same blocks took 3.5 ms. Ordinary stores, which the L2 can merge for a short while:
+// non-temporal ones lose that (order 3, 151 x 149, mixed: 73 against 106 us). Before, with the Gram sums on the
+// vector ALU in 4 x 4-node register tiles and 8-byte stores: 2.34 ms, and the assembly 2.80 ms; order 3 mixed
+// 142 us. Three wavefronts per SIMD: 2.17 ms against 2.23 ms for two (what the registers of order 4 give by
+// themselves) and for four.
 template <int P, typename T, int WAVES, bool RES, bool ACC = false>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVES > 1 ? 3 : 2)))
 void element_tiled_kernel(const SplitJob job, const Basis1D basisIn) {
   using O = Ord<P>;
   __shared__ WaveLDSTile<P, T> wl[WAVES];
@@ -840,14 +848,10 @@ __device__ __forceinline__ int find_job(const int *start, int n, int64_t x) {
 // A batch's element-once jobs of one order: counts = (jobs, units, staged blocks, staged residual entries)
 // in device memory (so a recorded graph replays any batch), unitStart[j] the first unit of job j, a unit
 // being WAVES * EPW elements. Persistent: workgroups stride over the units.
-// Two wavefronts per SIMD are requested explicitly: the persistent loop's state would otherwise push the
-// FP64 variants past 256 registers (one wavefront per SIMD); FP64 batch 56.6 ms against 59.3 ms with a few
-// registers spilled.
 template <int P, typename T, int WAVES, bool RES>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2))) void element_tiled_batch(const SplitJob *__restrict__ jobs,
-                                                                   const int *__restrict__ unitStart,
-                                                                   const int *__restrict__ counts,
-                                                                   const Basis1D basisIn) {
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(3)))
+void element_tiled_batch(const SplitJob *__restrict__ jobs, const int *__restrict__ unitStart,
+                         const int *__restrict__ counts, const Basis1D basisIn) {
   using O = Ord<P>;
   __shared__ WaveLDSTile<P, T> wl[WAVES];
   __shared__ Basis1D basis;
@@ -1267,8 +1271,6 @@ __device__ __forceinline__ void stage_stiffness_rows(WaveLDS<P, T> &W, const dou
     rows_chunk<P, T, JAC, CH, ALL_LANES>(W, gref, m, el, b, valid, count, c * CH, c == 0, Rx, Ry, where, emit);
   }
 }
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // MFMA form of the row-restricted stiffness (mixed precision, orders >= 3). For each chunk of 8 owned rows
 // of an element, the Gram sums are one product C = A B with
@@ -2021,52 +2023,64 @@ void launch_element_split(const SplitJob &job, const Basis1D &basis, int waves, 
   else go(std::integral_constant<int, kTiledWaves>{});
 }
 
-// Second pass of the element-once assembly: output dst[i] (C doubles from C * dst[i]) is the sum of the
-// staged contributions in slots ptr[i] .. ptr[i+1]-1, in slot order; zero if there are none. Lane t covers
-// component t % C of output t / C, so a wavefront reads consecutive slots.
+// Second pass of the element-once assembly, over 64-byte lines of the output (GatherList): 16-byte piece h of
+// line i is read, its unit's staged contributions are added in slot order, and it is stored. The four lanes of
+// a line store all of it, also the outputs that nothing is added to: a store of 32 bytes to a line that has left
+// the L2 costs about as much memory time as one of 128 (measured for scattered stores: 0.73 TB/s in pieces of
+// 32 bytes, 3.3 TB/s of 64, 5.3 TB/s of 128).
 template <int C>
-__device__ __forceinline__ void gather_one(const int *dst, const int *ptr, const double *stage, double *out, int64_t i,
-                                           int c, bool accumulate = false) {
-  const int k0 = ptr[i], k1 = ptr[i + 1];
-  double sum = 0;
-  for (int k = k0; k < k1; k++) sum += __builtin_nontemporal_load(stage + int64_t(C) * k + c);
-  double *o = out + int64_t(C) * dst[i] + c;
-  if (accumulate) sum += *o;
-  __builtin_nontemporal_store(sum, o);
+__device__ __forceinline__ void gather_one(const int *line, const int *ptr, const int *src, const double *stage,
+                                           double *out, int outputs, int64_t i, int h, bool accumulate = false) {
+  constexpr int U = 8 / C, H = C / 2;  // outputs per line, pieces per output
+  const int u = h / H, at = U * line[i] + u;
+  int k = ptr[U * i + u];
+  const int k1 = ptr[U * i + u + 1];
+  if (at >= outputs) return;
+  double2u *o = reinterpret_cast<double2u *>(out + int64_t(C) * at) + h % H;
+  double2u sum = *o;
+  if (k < k1 && src[k] < 0) {  // no contribution
+    if (!accumulate) sum = double2u{0, 0};
+    k++;
+  }
+  for (; k < k1; k++) sum += reinterpret_cast<const double2u *>(stage)[int64_t(H) * src[k] + h % H];
+  *o = sum;
 }
 
 template <int C>
-__global__ __launch_bounds__(256) void gather_shared(const int *dst, const int *ptr, const double *stage,
-                                                     double *out, int n, int accumulate) {
-  const int64_t total = int64_t(n) * C, stride = int64_t(gridDim.x) * 256;
+__global__ __launch_bounds__(256) void gather_shared(const int *line, const int *ptr, const int *src,
+                                                     const double *stage, double *out, int outputs, int n,
+                                                     int accumulate) {
+  const int64_t total = int64_t(n) * 4, stride = int64_t(gridDim.x) * 256;
   for (int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x; t < total; t += stride) {
-    gather_one<C>(dst, ptr, stage, out, t / C, int(t % C), accumulate != 0);
+    gather_one<C>(line, ptr, src, stage, out, outputs, t / 4, int(t % 4), accumulate != 0);
   }
 }
 
 template <int C>
-void launch_gather_shared(const int *dst, const int *ptr, const double *stage, double *out, int n, int accumulate,
-                          hipStream_t stream) {
-  const int64_t blocks = (int64_t(n) * C + 255) / 256;
+void launch_gather_shared(const int *line, const int *ptr, const int *src, const double *stage, double *out,
+                          int outputs, int n, int accumulate, hipStream_t stream) {
+  const int64_t blocks = (int64_t(n) * 4 + 255) / 256;
   if (n > 0) {
-    gather_shared<C><<<unsigned(std::min<int64_t>(blocks, 1 << 20)), 256, 0, stream>>>(dst, ptr, stage, out, n,
-                                                                                        accumulate);
+    gather_shared<C><<<unsigned(std::min<int64_t>(blocks, 1 << 20)), 256, 0, stream>>>(line, ptr, src, stage, out,
+                                                                                        outputs, n, accumulate);
   }
 }
 
-// The gathers of a batch's element-once jobs: C = 4, the staged blocks (outStart[j]: job j's first output
-// over all jobs, counts[2] in total), or C = 2, the staged residual entries (counts[3]; jobs without a
-// residual have none).
+// The gathers of a batch's element-once jobs: C = 4, the blocks' lines (lineStart[j]: job j's first line over all
+// jobs, counts[2] in total), or C = 2, the residual's (counts[3]; jobs without a residual have none).
 template <int C>
-__global__ __launch_bounds__(256) void gather_batch(const SplitJob *jobs, const int *outStart, const int *counts) {
+__global__ __launch_bounds__(256) void gather_batch(const SplitJob *jobs, const int *lineStart, const int *counts) {
   const int numJobs = counts[0];
-  const int64_t total = int64_t(counts[C == 4 ? 2 : 3]) * C, stride = int64_t(gridDim.x) * 256;
+  const int64_t total = int64_t(counts[C == 4 ? 2 : 3]) * 4, stride = int64_t(gridDim.x) * 256;
   for (int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x; t < total; t += stride) {
-    const int64_t i = t / C;
-    const int j = find_job(outStart, numJobs, i);
+    const int64_t i = t / 4;
+    const int j = find_job(lineStart, numJobs, i), h = int(t % 4);
     const SplitJob &job = jobs[j];
-    if (C == 4) gather_one<4>(job.gdst, job.gptr, job.stage, job.values, i - outStart[j], int(t % C));
-    else gather_one<2>(job.rdst, job.rptr, job.rstage, job.residual, i - outStart[j], int(t % C));
+    if (C == 4) {
+      gather_one<4>(job.gline, job.gptr, job.gsrc, job.stage, job.values, job.numBlocks, i - lineStart[j], h);
+    } else {
+      gather_one<2>(job.rline, job.rptr, job.rsrc, job.rstage, job.residual, job.numNodes, i - lineStart[j], h);
+    }
   }
 }
 
@@ -2082,8 +2096,12 @@ void launch_split(const SplitJob &job, const Basis1D &basis, int precision, int 
     if (res) launch_element_split<P, double, true>(job, basis, waves, s);
     else launch_element_split<P, double, false>(job, basis, waves, s);
   }
-  launch_gather_shared<4>(job.gdst, job.gptr, job.stage, job.values, job.numGather, job.accumulate, s);
-  if (res) launch_gather_shared<2>(job.rdst, job.rptr, job.rstage, job.residual, job.numRgather, job.accumulate, s);
+  launch_gather_shared<4>(job.gline, job.gptr, job.gsrc, job.stage, job.values, job.numBlocks, job.numGather,
+                          job.accumulate, s);
+  if (res) {
+    launch_gather_shared<2>(job.rline, job.rptr, job.rsrc, job.rstage, job.residual, job.numNodes, job.numRgather,
+                            job.accumulate, s);
+  }
 }
 
 template <int P, bool RES, bool JAC>
@@ -2192,10 +2210,12 @@ SplitJob make_split_job(const fem_plan *p, const double *states, const double *c
   j.conn = p->dConn;
   j.code = p->dCode;
   j.rcode = p->dRcode;
-  j.gdst = p->dGdst;
+  j.gline = p->dGline;
   j.gptr = p->dGptr;
-  j.rdst = p->dRdst;
+  j.gsrc = p->dGsrc;
+  j.rline = p->dRline;
   j.rptr = p->dRptr;
+  j.rsrc = p->dRsrc;
   j.states = states;
   j.coords = coords;
   j.residual = residual;
@@ -2267,7 +2287,8 @@ int alloc_doubles(int64_t n, double **d, int64_t &bytes) {
 void free_plan_arrays(fem_plan *p) {
   void *ptrs[] = {p->dVisitConn, p->dVisitEid, p->dNodeLrow, p->dRows,  p->dRowLbase, p->dRuns,  p->dColourOff,
                   p->dPartDesc,  p->dRank,     p->dJob,      p->dJobStart, p->dConn,   p->dCode,  p->dRcode,
-                  p->dGdst,      p->dGptr,     p->dRdst,     p->dRptr,   p->dStage,    p->dRstage};
+                  p->dGline,     p->dGptr,     p->dGsrc,     p->dRline,  p->dRptr,     p->dRsrc,  p->dStage,
+                  p->dRstage};
   for (void *q : ptrs) {
     if (q) (void)hipFree(q);
   }
@@ -2464,20 +2485,24 @@ int create_plan(int order, int numNodes, int numElements, const int *connPtr, co
     for (int e = 0; e < numElements; e++) std::copy(conn + connPtr[e], conn + connPtr[e] + N, c.begin() + size_t(e) * N);
     SplitHost sp;
     if (build_split_host(order, numNodes, numElements, c.data(), rowp, h.rank, h.numBlocks, sp) == FEM_OK) {
+      GatherList gl, rl;
+      plan_gather(h.numBlocks, 2, sp.code, sp.dst, sp.ptr, gl);
+      plan_gather(numNodes, 4, sp.rcode, sp.rdst, sp.rptr, rl);
       h = PlanHost();  // the owner tables are on the device; release their host copies first
       if ((rc = upload(c, &p->dConn, bytes)) || (rc = upload(sp.code, &p->dCode, bytes)) ||
-          (rc = upload(sp.rcode, &p->dRcode, bytes)) || (rc = upload(sp.dst, &p->dGdst, bytes)) ||
-          (rc = upload(sp.ptr, &p->dGptr, bytes)) || (rc = upload(sp.rdst, &p->dRdst, bytes)) ||
-          (rc = upload(sp.rptr, &p->dRptr, bytes)) || (rc = alloc_doubles(4 * sp.slots, &p->dStage, bytes)) ||
-          (rc = alloc_doubles(2 * sp.rslots, &p->dRstage, bytes))) {
+          (rc = upload(sp.rcode, &p->dRcode, bytes)) || (rc = upload(gl.line, &p->dGline, bytes)) ||
+          (rc = upload(gl.ptr, &p->dGptr, bytes)) || (rc = upload(gl.src, &p->dGsrc, bytes)) ||
+          (rc = upload(rl.line, &p->dRline, bytes)) || (rc = upload(rl.ptr, &p->dRptr, bytes)) ||
+          (rc = upload(rl.src, &p->dRsrc, bytes)) || (rc = alloc_doubles(4 * gl.slots, &p->dStage, bytes)) ||
+          (rc = alloc_doubles(2 * rl.slots, &p->dRstage, bytes))) {
         free_plan_arrays(p);
         delete p;
         return rc;
       }
-      p->numGather = int(sp.dst.size());
-      p->numRgather = int(sp.rdst.size());
-      p->numSlots = sp.slots;
-      p->numRslots = sp.rslots;
+      p->numGather = int(gl.line.size());
+      p->numRgather = int(rl.line.size());
+      p->numSlots = gl.slots;
+      p->numRslots = rl.slots;
     } else {
       clear_error();
     }

@@ -489,6 +489,56 @@ int build_split_host(int order, int numNodes, int numElements, const int *conn, 
   return split_outputs(int64_t(numElements) * N, numNodes, nodeDest, out.rcode, out.rdst, out.rptr, out.rslots);
 }
 
+void plan_gather(int64_t outputs, int unitsPerLine, std::vector<int> &code, const std::vector<int> &dst,
+                 const std::vector<int> &ptr, GatherList &out) {
+  // first[k]: the output whose first contribution has slot k of the input tables, else -1
+  std::vector<int> first(size_t(ptr.back()), -1);
+  for (size_t i = 0; i < dst.size(); i++) {
+    if (ptr[i + 1] > ptr[i]) first[size_t(ptr[i])] = dst[i];
+  }
+  // Renumber the other contributions' slots in contribution order (chunk counts, prefix sums, assignment).
+  constexpr int64_t kChunk = 1 << 18;
+  const int64_t n = int64_t(code.size()), chunks = (n + kChunk - 1) / kChunk;
+  std::vector<int> start(size_t(chunks) + 1, 0), slot(first.size(), -1);
+  auto staged = [&](int v) { return v >= outputs && first[size_t(v - outputs)] < 0; };
+  parallel_for(chunks, [&](int64_t b, int64_t e) {
+    for (int64_t c = b; c < e; c++) {
+      int count = 0;
+      for (int64_t i = c * kChunk; i < std::min(n, (c + 1) * kChunk); i++) count += staged(code[size_t(i)]);
+      start[size_t(c) + 1] = count;
+    }
+  });
+  for (int64_t c = 0; c < chunks; c++) start[size_t(c) + 1] += start[size_t(c)];
+  out.slots = start[size_t(chunks)];
+  parallel_for(chunks, [&](int64_t b, int64_t e) {
+    for (int64_t c = b; c < e; c++) {
+      int next = start[size_t(c)];
+      for (int64_t i = c * kChunk; i < std::min(n, (c + 1) * kChunk); i++) {
+        int &v = code[size_t(i)];
+        if (staged(v)) {
+          slot[size_t(v - outputs)] = next;
+          v = int(outputs) + next++;
+        } else if (v >= outputs) {
+          v = first[size_t(v - outputs)];
+        }
+      }
+    }
+  });
+  out.line.clear();
+  out.ptr.assign(1, 0);
+  out.src.clear();
+  out.src.reserve(size_t(out.slots));
+  for (size_t i = 0; i < dst.size(); i++) {
+    const int line = dst[i] / unitsPerLine, unit = dst[i] % unitsPerLine;
+    if (out.line.empty() || out.line.back() != line) out.line.push_back(line);
+    // units of the line before this one without an entry of their own have empty ranges
+    out.ptr.resize((out.line.size() - 1) * unitsPerLine + unit + 1, int(out.src.size()));
+    if (ptr[i + 1] == ptr[i]) out.src.push_back(-1);
+    for (int k = ptr[i] + 1; k < ptr[i + 1]; k++) out.src.push_back(slot[size_t(k)]);
+  }
+  out.ptr.resize(out.line.size() * unitsPerLine + 1, int(out.src.size()));
+}
+
 }  // namespace fem
 
 using namespace fem;

@@ -66,7 +66,7 @@ struct PlanHost {
   int maxPartVisits = 0;
 };
 
-// Element-once assembly tables (orders 3-4). Every output (a BSR block, or a node's residual pair) is either
+// Element-once tables (orders 3-4). Every output (a BSR block, or a node's residual pair) is either
 // exclusive, formed by exactly one (element, node[, node]) contribution, or not. An exclusive output is
 // stored by its one contributor; the contributions to any other output go to slots of a staging array,
 // grouped by output, and a gather pass stores each such output as the sum of its slots in slot order (zero
@@ -87,6 +87,20 @@ struct SplitHost {
 // plan's column ranks. Returns FEM_ERR_UNSUPPORTED if the codes would not fit in an int.
 int build_split_host(int order, int numNodes, int numElements, const int *conn, const int *rowp,
                      const std::vector<uint8_t> &rank, int64_t numBlocks, SplitHost &out);
+
+// What a plan's element-once assembly does with those tables. An output's first contribution is stored in place,
+// like an exclusive one; the others go to staging slots, numbered in contribution order (so an element's are
+// contiguous), and the gather adds them. It works on lines of 64 bytes of the output array (unitsPerLine
+// outputs each) that hold at least one output to add to: line l's unit u is output unitsPerLine * line[l] + u and
+// gets the slots src[ptr[unitsPerLine * l + u]] .. src[ptr[unitsPerLine * l + u + 1] - 1] added in that
+// order; a slot of -1 stands for an output without contributions, which is stored as zero.
+struct GatherList {
+  std::vector<int> line, ptr, src;
+  int64_t slots = 0;
+};
+// Rewrites code (destinations below `outputs`, else outputs + slot; dst / ptr as in SplitHost) accordingly.
+void plan_gather(int64_t outputs, int unitsPerLine, std::vector<int> &code, const std::vector<int> &dst,
+                 const std::vector<int> &ptr, GatherList &out);
 
 // partScale (0, 1] scales the part budgets (blocks, rows, visits) below the kernel's maxima: smaller
 // parts give small meshes more workgroups at the price of more elements recomputed on part boundaries.
@@ -140,10 +154,11 @@ struct fem_plan {
   int *dConn = nullptr;      // [E][N]
   int *dCode = nullptr;      // [E][N][N]
   int *dRcode = nullptr;     // [E][N]
-  int *dGdst = nullptr, *dGptr = nullptr, *dRdst = nullptr, *dRptr = nullptr;
+  int *dGline = nullptr, *dGptr = nullptr, *dGsrc = nullptr;  // GatherList of the blocks (2 per line)
+  int *dRline = nullptr, *dRptr = nullptr, *dRsrc = nullptr;  // and of the residual entries (4 per line)
   double *dStage = nullptr;  // [4 * slots]
   double *dRstage = nullptr; // [2 * rslots]
-  int numGather = 0, numRgather = 0;
+  int numGather = 0, numRgather = 0;    // gathered lines
   int64_t numSlots = 0, numRslots = 0;  // staged contributions: blocks, residual entries
   double partScale = 1.0;    // part budgets relative to the kernel's (FEM_PLAN_AUTOTUNE picks it)
   double tunedSeconds = 0;   // measured assembly time of the chosen build (autotuned plans)

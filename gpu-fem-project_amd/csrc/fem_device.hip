@@ -430,15 +430,15 @@ struct ElemArgs {
   Material mat;
 };
 
-template <int P, typename T, int WAVES, bool RES, bool JAC, bool ATOMIC>
+template <int P, typename T, int WAVES, bool RES, bool ATOMIC>
 __global__ __launch_bounds__(WAVES * 64) void element_kernel(const ElemArgs args) {
   using O = Ord<P>;
   constexpr int N = O::N;
   __shared__ WaveLDS<P, T> wl[WAVES];
   __shared__ Basis1D basis;
   __shared__ double2 gref[O::Q * O::N];
-  __shared__ double stK[JAC ? WAVES : 1][4][64];  // Jacobian emission: each lane's block, by component
-  __shared__ int stAt[JAC ? WAVES : 1][64];        // and its destination (negative: none)
+  __shared__ double stK[WAVES][4][64];  // emission: each lane's block, by component
+  __shared__ int stAt[WAVES][64];        // and its destination (negative: none)
   copy_basis(basis, args.basis);
   fill_gref<P>(gref, args.basis);
   __syncthreads();
@@ -461,44 +461,30 @@ __global__ __launch_bounds__(WAVES * 64) void element_kernel(const ElemArgs args
   const int *mel = args.map + int64_t(eid) * N * N;
   double Rx, Ry;
   auto where = [&](int row, int col) __attribute__((always_inline)) { return mel[row * N + col]; };
-  auto emit = [&](int at, const double(&k)[4]) __attribute__((always_inline)) {
-    double *blk = args.values + at;
-    if (ATOMIC) {
+  // Row-major emission: every row of K_e in chunks, so the lanes of an element hold neighbouring blocks of
+  // one BSR row. The blocks then pass through LDS so that each add instruction covers the four
+  // components of 16 blocks (lanes 4i..4i+3 take block i), 32 contiguous bytes per block.
+  if (valid) W.orow[el][idx] = (unsigned char)idx;
+  wave_sync();
+  auto emitRows = [&](int at, const double(&k)[4]) __attribute__((always_inline)) {
+    stAt[wave][lane] = at;
 #pragma unroll
-      for (int c = 0; c < 4; c++) unsafeAtomicAdd(blk + c, k[c]);
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; c++) blk[c] += k[c];
-    }
-  };
-  if constexpr (JAC) {
-    // Row-major emission: every row of K_e in chunks, so the lanes of an element hold neighbouring blocks of
-    // one BSR row. The blocks then pass through LDS so that each add instruction covers the four
-    // components of 16 blocks (lanes 4i..4i+3 take block i), 32 contiguous bytes per block.
-    if (valid) W.orow[el][idx] = (unsigned char)idx;
+    for (int c = 0; c < 4; c++) stK[wave][c][lane] = k[c];
     wave_sync();
-    auto emitRows = [&](int at, const double(&k)[4]) __attribute__((always_inline)) {
-      stAt[wave][lane] = at;
+    const int c = lane & 3;
 #pragma unroll
-      for (int c = 0; c < 4; c++) stK[wave][c][lane] = k[c];
-      wave_sync();
-      const int c = lane & 3;
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int src = (lane >> 2) + 16 * r;
-        const int a = stAt[wave][src];
-        if (a >= 0) {
-          double *blk = args.values + a + c;
-          if (ATOMIC) unsafeAtomicAdd(blk, stK[wave][c][src]);
-          else *blk += stK[wave][c][src];
-        }
+    for (int r = 0; r < 4; r++) {
+      const int src = (lane >> 2) + 16 * r;
+      const int a = stAt[wave][src];
+      if (a >= 0) {
+        double *blk = args.values + a + c;
+        if (ATOMIC) unsafeAtomicAdd(blk, stK[wave][c][src]);
+        else *blk += stK[wave][c][src];
       }
-      wave_sync();  // the next row restages into the same slots
-    };
-    stage_stiffness_rows<P, T, JAC, true>(W, gref, args.mat, el, idx, valid, N, N, Rx, Ry, where, emitRows);
-  } else {
-    stage_stiffness<P, T, JAC>(W, gref, args.mat, el, idx, valid, Rx, Ry, where, emit);
-  }
+    }
+    wave_sync();  // the next row restages into the same slots
+  };
+  stage_stiffness_rows<P, T, true, true>(W, gref, args.mat, el, idx, valid, N, N, Rx, Ry, where, emitRows);
   if (RES && valid) {
     double *r = args.residual + 2 * int64_t(node);
     if (ATOMIC) {
@@ -869,6 +855,191 @@ void element_tiled_batch(const SplitJob *__restrict__ jobs, const int *__restric
   }
 }
 
+// ---- residual alone, by lines of nodes ------------------------------------------------------------------
+// The residual is bound by memory (48 bytes per node and 4 per node reference against 8 N fused multiply-adds
+// per point), so its arithmetic is sum-factorised: lane (el, k) holds line k of an element's NP x NP grid, NP
+// elements-lines per element and floor(64 / NP) elements per wavefront. Forward, lane (el, ay) contracts its
+// nodes along x for every qx, the results are exchanged through LDS, and lane (el, qx) contracts along y: it
+// then holds the derivatives at its NP quadrature points. The stresses, pulled back to the reference element
+// (P = s sigma J^-T), go back the same way: R_a = sum_q P(q) g_a(q). Basis values are uniform (scalar registers).
+template <int P>
+struct LineOrd {
+  static constexpr int NP = P + 1, N = NP * NP;
+  static constexpr int EPW = 64 / NP;
+  // Exchange: 4 doubles per (line, point); rows and elements an odd number of 16-byte units apart.
+  static constexpr int ROW = 4 * NP + 2;
+  static constexpr int EL = NP * ROW + (NP % 2 == 0 ? 2 : 0);
+};
+
+struct __align__(16) Quad {
+  double2 a, b;
+};
+
+// Derivatives (d/dxi of both components, then d/deta) at lane (el, qx)'s points of the nodal field f of lane
+// (el, ay)'s nodes. `ex` is the element's exchange area.
+template <int P>
+__device__ __forceinline__ void line_gradients(double *ex, const Basis1D &B, int line, bool write,
+                                               const double2 (&f)[P + 1], double (&G)[P + 1][4]) {
+  using O = LineOrd<P>;
+  constexpr int NP = O::NP;
+  wave_sync();  // the exchange area's previous readers are done
+#pragma unroll
+  for (int qx = 0; qx < NP; qx++) {
+    Quad t{make_double2(0, 0), make_double2(0, 0)};
+#pragma unroll
+    for (int ax = 0; ax < NP; ax++) {
+      t.a.x = fma(B.phi[ax][qx], f[ax].x, t.a.x);
+      t.a.y = fma(B.phi[ax][qx], f[ax].y, t.a.y);
+      t.b.x = fma(B.dphi[ax][qx], f[ax].x, t.b.x);
+      t.b.y = fma(B.dphi[ax][qx], f[ax].y, t.b.y);
+    }
+    if (write) *reinterpret_cast<Quad *>(ex + line * O::ROW + 4 * qx) = t;
+  }
+  wave_sync();
+#pragma unroll
+  for (int qy = 0; qy < NP; qy++) G[qy][0] = G[qy][1] = G[qy][2] = G[qy][3] = 0;
+#pragma unroll
+  for (int ay = 0; ay < NP; ay++) {
+    const Quad t = *reinterpret_cast<const Quad *>(ex + ay * O::ROW + 4 * line);
+#pragma unroll
+    for (int qy = 0; qy < NP; qy++) {
+      G[qy][0] = fma(B.phi[ay][qy], t.b.x, G[qy][0]);
+      G[qy][1] = fma(B.phi[ay][qy], t.b.y, G[qy][1]);
+      G[qy][2] = fma(B.dphi[ay][qy], t.a.x, G[qy][2]);
+      G[qy][3] = fma(B.dphi[ay][qy], t.a.y, G[qy][3]);
+    }
+  }
+}
+
+// Residual of lane (el, ay)'s nodes from their coordinates and displacements. NL: the NONLINEAR (Green) strain.
+// Every lane of the wavefront calls it; `write` masks the lanes past the wavefront's elements.
+template <int P, bool NL>
+__device__ __forceinline__ void line_residual(double *ex, const Basis1D &B, const Material &m, int line, bool write,
+                                              const double2 (&xy)[P + 1], const double2 (&uv)[P + 1],
+                                              double2 (&R)[P + 1]) {
+  using O = LineOrd<P>;
+  constexpr int NP = O::NP;
+  double J[NP][4], U[NP][4];
+  line_gradients<P>(ex, B, line, write, xy, J);
+  line_gradients<P>(ex, B, line, write, uv, U);
+  double wx = B.w[0];
+#pragma unroll
+  for (int k = 1; k < NP; k++) wx = line == k ? B.w[k] : wx;
+#pragma unroll
+  for (int qy = 0; qy < NP; qy++) {
+    const double J00 = J[qy][0], J10 = J[qy][1], J01 = J[qy][2], J11 = J[qy][3];
+    const double detJ = J00 * J11 - J01 * J10;
+    const double inv = 1.0 / detJ;
+    const double i00 = J11 * inv, i01 = -J01 * inv, i10 = -J10 * inv, i11 = J00 * inv;
+    const double G00 = U[qy][0] * i00 + U[qy][2] * i10;
+    const double G01 = U[qy][0] * i01 + U[qy][2] * i11;
+    const double G10 = U[qy][1] * i00 + U[qy][3] * i10;
+    const double G11 = U[qy][1] * i01 + U[qy][3] * i11;
+    const double s = (wx * B.w[qy]) * detJ * m.t;
+    double f00, f01, f10, f11;  // s sigma (NL: s F S)
+    if (NL) {
+      const double exx = G00 + 0.5 * (G00 * G00 + G10 * G10);
+      const double eyy = G11 + 0.5 * (G01 * G01 + G11 * G11);
+      const double exy = 0.5 * (G01 + G10 + G00 * G01 + G10 * G11);
+      const double tr = exx + eyy;
+      const double Sxx = 2 * m.mu * exx + m.lambda * tr, Syy = 2 * m.mu * eyy + m.lambda * tr, Sxy = 2 * m.mu * exy;
+      f00 = s * ((1 + G00) * Sxx + G01 * Sxy);
+      f01 = s * ((1 + G00) * Sxy + G01 * Syy);
+      f10 = s * (G10 * Sxx + (1 + G11) * Sxy);
+      f11 = s * (G10 * Sxy + (1 + G11) * Syy);
+    } else {
+      const double tr = G00 + G11;
+      f00 = s * (2 * m.mu * G00 + m.lambda * tr);
+      f11 = s * (2 * m.mu * G11 + m.lambda * tr);
+      f01 = f10 = s * (m.mu * (G01 + G10));
+    }
+    U[qy][0] = f00 * i00 + f01 * i01;  // reference direction xi
+    U[qy][1] = f10 * i00 + f11 * i01;
+    U[qy][2] = f00 * i10 + f01 * i11;  // eta
+    U[qy][3] = f10 * i10 + f11 * i11;
+  }
+  wave_sync();
+#pragma unroll
+  for (int ay = 0; ay < NP; ay++) {
+    Quad t{make_double2(0, 0), make_double2(0, 0)};
+#pragma unroll
+    for (int qy = 0; qy < NP; qy++) {
+      t.a.x = fma(B.phi[ay][qy], U[qy][0], t.a.x);
+      t.a.y = fma(B.phi[ay][qy], U[qy][1], t.a.y);
+      t.b.x = fma(B.dphi[ay][qy], U[qy][2], t.b.x);
+      t.b.y = fma(B.dphi[ay][qy], U[qy][3], t.b.y);
+    }
+    if (write) *reinterpret_cast<Quad *>(ex + ay * O::ROW + 4 * line) = t;
+  }
+  wave_sync();
+#pragma unroll
+  for (int ax = 0; ax < NP; ax++) R[ax] = make_double2(0, 0);
+#pragma unroll
+  for (int qx = 0; qx < NP; qx++) {
+    const Quad t = *reinterpret_cast<const Quad *>(ex + line * O::ROW + 4 * qx);
+#pragma unroll
+    for (int ax = 0; ax < NP; ax++) {
+      R[ax].x = fma(B.dphi[ax][qx], t.a.x, fma(B.phi[ax][qx], t.b.x, R[ax].x));
+      R[ax].y = fma(B.dphi[ax][qx], t.a.y, fma(B.phi[ax][qx], t.b.y, R[ax].y));
+    }
+  }
+}
+
+// Drop-in residual (fem_residual, fem_residual_nonlinear): FP64 atomics, which bound it. Where an element's last
+// nodes of its lines are the first ones of the next element of the wavefront (consecutive elements along x), it adds
+// that element's share to its own, a third less to add at order 2. The residuals pass through LDS once more so
+// that neighbouring lanes add the two components of an element's consecutive nodes. 351 x 350 order 2: 20 us, of
+// which the adds are most (31 us without the merge; 42 us in the element kernel it replaces).
+constexpr int kLineWaves = 4;
+template <int P, bool NL>
+__global__ __launch_bounds__(kLineWaves * 64) void residual_kernel(const ElemArgs args) {
+  using O = LineOrd<P>;
+  constexpr int NP = O::NP, N = O::N;
+  __shared__ __align__(16) double exAll[kLineWaves][O::EPW * O::EL];
+  __shared__ int idAll[kLineWaves][O::EPW * N];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int64_t first = (int64_t(xcd_block()) * kLineWaves + wave) * O::EPW;
+  if (first >= args.count) return;  // whole wavefront
+  double *ex = exAll[wave];
+  int *ids = idAll[wave];
+  const int el = min(lane / NP, O::EPW - 1), line = lane % NP;
+  const bool write = lane < O::EPW * NP;
+  const int count = int(min<int64_t>(O::EPW, args.count - first));
+  const int *conn = args.conn + args.connPtr[first + min(el, count - 1)] + line * NP;
+  double2 xy[NP], uv[NP], R[NP];
+  int node[NP];
+#pragma unroll
+  for (int k = 0; k < NP; k++) {
+    node[k] = conn[k];
+    xy[k] = *reinterpret_cast<const double2 *>(args.coords + 2 * int64_t(node[k]));
+    uv[k] = *reinterpret_cast<const double2 *>(args.states + 2 * int64_t(node[k]));
+  }
+  line_residual<P, NL>(ex + el * O::EL, args.basis, args.mat, line, write, xy, uv, R);
+  {
+    const int right = __shfl_down(node[0], NP), left = __shfl_up(node[P], NP);
+    const double rx = __shfl_down(R[0].x, NP), ry = __shfl_down(R[0].y, NP);
+    if (write && el + 1 < count && right == node[P]) {
+      R[P].x += rx;
+      R[P].y += ry;
+    }
+    if (write && el > 0 && el < count && left == node[0]) node[0] = -1;  // added by the element before
+  }
+  if (write) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) ids[el * N + line * NP + k] = node[k];
+  }
+  wave_sync();
+  if (write) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) reinterpret_cast<double2 *>(ex)[el * N + line * NP + k] = R[k];
+  }
+  wave_sync();
+  for (int k = lane; k < 2 * N * count; k += 64) {
+    const int id = ids[k >> 1];
+    if (id >= 0) unsafeAtomicAdd(args.residual + 2 * int64_t(id) + (k & 1), ex[k]);
+  }
+}
+
 // ---- NONLINEAR (Green) strain: element-parallel drop-in paths ------------------------------------------
 // The reference's kernels with GreenStrainType::NONLINEAR (element/FEKernels.h:286-315, 585-1006): Green
 // strain E = (Ux + Ux^T + Ux^T Ux) / 2, S = 2 mu E + lambda tr(E) I, weak residual s F S with F = I + Ux
@@ -951,11 +1122,11 @@ __device__ __forceinline__ void stage_geometry_nl(WaveLDSNL<P> &W, const Basis1D
   g[19] = 0;
 }
 
-// Lane (el, b): residual of node b and (JAC) the blocks K(a, b) of every row a, in chunks of CH rows; the
+// Lane (el, b): residual of node b and the blocks K(a, b) of every row a, in chunks of CH rows; the
 // gradients of the chunk's rows come through the per-wave LDS one quadrature point at a time. All lanes of
 // the wavefront must call this; `valid` masks the lane's writes. Every lane calls emit(at, k) for every row,
 // in step, with a negative destination when it has none (so emit may exchange values across lanes).
-template <int P, bool JAC, typename Where, typename Emit>
+template <int P, typename Where, typename Emit>
 __device__ __forceinline__ void stage_stiffness_nl(WaveLDSNL<P> &W, const double2 *gref, const Material &m, int el,
                                                    int b, bool valid, double &Rx, double &Ry, Where &&where,
                                                    Emit &&emit) {
@@ -967,7 +1138,7 @@ __device__ __forceinline__ void stage_stiffness_nl(WaveLDSNL<P> &W, const double
   Rx = 0;
   Ry = 0;
 #pragma unroll 1
-  for (int c0 = 0; c0 < (JAC ? N : 1); c0 += CH) {
+  for (int c0 = 0; c0 < N; c0 += CH) {
     double A[CH][3], Tm[CH][4], H[CH];
 #pragma unroll
     for (int j = 0; j < CH; j++) {
@@ -985,58 +1156,55 @@ __device__ __forceinline__ void stage_stiffness_nl(WaveLDSNL<P> &W, const double
         Rx += g[5] * nx + g[6] * ny;
         Ry += g[7] * nx + g[8] * ny;
       }
-      if (JAC) {
-        const double s = g[4];
-        const double px = g[9] * nx + g[10] * ny, py = g[11] * nx + g[12] * ny;
-        const double spx = s * px, spy = s * py;
-        const double qx = g[16] * nx + g[17] * ny, qy = g[17] * nx + g[18] * ny;
-        if (valid) {
-          W.pub[el][b][0] = make_double2(nx, ny);
-          W.pub[el][b][1] = make_double2(px, py);
-        }
-        wave_sync();
-#pragma unroll
-        for (int j = 0; j < CH; j++) {
-          const int a = c0 + j < N ? c0 + j : N - 1;
-          const double2 na = W.pub[elc][a][0], pa = W.pub[elc][a][1];
-          const double sd = s * (na.x * nx + na.y * ny);
-          A[j][0] = fma(sd, g[13], A[j][0]);
-          A[j][1] = fma(sd, g[14], A[j][1]);
-          A[j][2] = fma(sd, g[15], A[j][2]);
-          Tm[j][0] = fma(pa.x, spx, Tm[j][0]);
-          Tm[j][1] = fma(pa.x, spy, Tm[j][1]);
-          Tm[j][2] = fma(pa.y, spx, Tm[j][2]);
-          Tm[j][3] = fma(pa.y, spy, Tm[j][3]);
-          H[j] = fma(na.x, qx, fma(na.y, qy, H[j]));
-        }
-        wave_sync();  // the next point republishes into the same slots
+      const double s = g[4];
+      const double px = g[9] * nx + g[10] * ny, py = g[11] * nx + g[12] * ny;
+      const double spx = s * px, spy = s * py;
+      const double qx = g[16] * nx + g[17] * ny, qy = g[17] * nx + g[18] * ny;
+      if (valid) {
+        W.pub[el][b][0] = make_double2(nx, ny);
+        W.pub[el][b][1] = make_double2(px, py);
       }
-    }
-    if (JAC) {  // every lane calls emit for every row, in step (negative destination: none)
-      int at[CH];
-#pragma unroll
-      for (int j = 0; j < CH; j++) at[j] = valid && c0 + j < N ? where(c0 + j, b) : -1;
+      wave_sync();
 #pragma unroll
       for (int j = 0; j < CH; j++) {
-        if (c0 + j >= N) break;
-        // K_ik = mu A_ik + mu T_ki + lambda T_ik + delta_ik H, T_ik = sum_q s (F n_a)_i (F n_b)_k
-        const double k[4] = {mu * A[j][0] + (mu + lam) * Tm[j][0] + H[j], mu * A[j][1] + mu * Tm[j][2] + lam * Tm[j][1],
-                             mu * A[j][1] + mu * Tm[j][1] + lam * Tm[j][2], mu * A[j][2] + (mu + lam) * Tm[j][3] + H[j]};
-        emit(at[j], k);
+        const int a = c0 + j < N ? c0 + j : N - 1;
+        const double2 na = W.pub[elc][a][0], pa = W.pub[elc][a][1];
+        const double sd = s * (na.x * nx + na.y * ny);
+        A[j][0] = fma(sd, g[13], A[j][0]);
+        A[j][1] = fma(sd, g[14], A[j][1]);
+        A[j][2] = fma(sd, g[15], A[j][2]);
+        Tm[j][0] = fma(pa.x, spx, Tm[j][0]);
+        Tm[j][1] = fma(pa.x, spy, Tm[j][1]);
+        Tm[j][2] = fma(pa.y, spx, Tm[j][2]);
+        Tm[j][3] = fma(pa.y, spy, Tm[j][3]);
+        H[j] = fma(na.x, qx, fma(na.y, qy, H[j]));
       }
+      wave_sync();  // the next point republishes into the same slots
+    }
+    // every lane calls emit for every row, in step (negative destination: none)
+    int at[CH];
+#pragma unroll
+    for (int j = 0; j < CH; j++) at[j] = valid && c0 + j < N ? where(c0 + j, b) : -1;
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      if (c0 + j >= N) break;
+      // K_ik = mu A_ik + mu T_ki + lambda T_ik + delta_ik H, T_ik = sum_q s (F n_a)_i (F n_b)_k
+      const double k[4] = {mu * A[j][0] + (mu + lam) * Tm[j][0] + H[j], mu * A[j][1] + mu * Tm[j][2] + lam * Tm[j][1],
+                           mu * A[j][1] + mu * Tm[j][1] + lam * Tm[j][2], mu * A[j][2] + (mu + lam) * Tm[j][3] + H[j]};
+      emit(at[j], k);
     }
   }
 }
 
-template <int P, int WAVES, bool RES, bool JAC>
+template <int P, int WAVES, bool RES>
 __global__ __launch_bounds__(WAVES * 64) void element_kernel_nl(const ElemArgs args) {
   using O = Ord<P>;
   constexpr int N = O::N;
   __shared__ WaveLDSNL<P> wl[WAVES];
   __shared__ Basis1D basis;
   __shared__ double2 gref[O::Q * O::N];
-  __shared__ double stK[JAC ? WAVES : 1][4][64];  // Jacobian emission staging, as in element_kernel
-  __shared__ int stAt[JAC ? WAVES : 1][64];
+  __shared__ double stK[WAVES][4][64];  // emission staging, as in element_kernel
+  __shared__ int stAt[WAVES][64];
   copy_basis(basis, args.basis);
   fill_gref<P>(gref, args.basis);
   __syncthreads();
@@ -1074,7 +1242,7 @@ __global__ __launch_bounds__(WAVES * 64) void element_kernel_nl(const ElemArgs a
     }
     wave_sync();
   };
-  stage_stiffness_nl<P, JAC>(W, gref, args.mat, el, idx, valid, Rx, Ry, where, emit);
+  stage_stiffness_nl<P>(W, gref, args.mat, el, idx, valid, Rx, Ry, where, emit);
   if (RES && valid) {
     double *r = args.residual + 2 * int64_t(node);
     unsafeAtomicAdd(r, Rx);
@@ -1102,6 +1270,7 @@ struct MeshJob {
   int numParts, numColours;
   int accumulate;  // 1: the write-out adds to the outputs (+=) instead of storing them
   int pad_;
+  const uint16_t *visitRow;  // residual-only plans: [visits*N] part-local row of each visit's nodes, or kNoRow
 };
 
 struct OwnerArgs {
@@ -1654,6 +1823,82 @@ __device__ __forceinline__ void zero_planes(double *acc, int nb) {
   }
 }
 
+// Residual-only plans: one workgroup per part, by lines of nodes, LDS sums per owned row, one store per row.
+// Bound by latency (701 x 699 order 2: VALU 40% and LDS 37% busy, 2.1 TB/s): 54 us against 148 for the kernel that
+// formed each node's gradient at every point (lane (el, node)) and looked the rows up per node; 67 us without the
+// loads running ahead and with parts of 1024 rows.
+template <int P, int MAXR>
+__global__ __launch_bounds__(kLineWaves * 64) void residual_part_kernel(const OwnerArgs args) {
+  using O = LineOrd<P>;
+  constexpr int NP = O::NP, N = O::N, THREADS = kLineWaves * 64;
+  __shared__ __align__(16) double exAll[kLineWaves][O::EPW * O::EL];
+  __shared__ __align__(16) double racc[2 * MAXR];
+  const MeshJob &J = args.jobs[0];
+  const int per = int(gridDim.x) / 8;  // contiguous parts per XCD, as in owner_kernel
+  const int part = int(blockIdx.x % 8) * per + int(blockIdx.x / 8);
+  if (part >= args.totalParts) return;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const PartDesc d = part_desc(J, part);
+  const Material mat = job_material(J);
+  for (int i = threadIdx.x; i < d.nr; i += THREADS) reinterpret_cast<double2 *>(racc)[i] = make_double2(0, 0);
+  __syncthreads();
+  const int el = min(lane / NP, O::EPW - 1), line = lane % NP;
+  const bool write = lane < O::EPW * NP;
+  double *ex = exAll[wave] + el * O::EL;
+  // Loads run ahead of the arithmetic: node ids two batches, nodes one. Indices are clamped into the part.
+  auto load_ids = [&](int v, int (&node)[NP], int (&row)[NP]) __attribute__((always_inline)) {
+    const int64_t at = int64_t(d.e0 + min(v + el, d.ne - 1)) * N + line * NP;
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      node[k] = gmem(J.visitConn)[at + k];
+      row[k] = gmem(J.visitRow)[at + k];
+    }
+  };
+  auto load_nodes = [&](const int (&node)[NP], double2 (&xy)[NP], double2 (&uv)[NP]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      xy[k] = gmem(reinterpret_cast<const double2 *>(J.coords))[node[k]];
+      uv[k] = gmem(reinterpret_cast<const double2 *>(J.states))[node[k]];
+    }
+  };
+  constexpr int STEP = kLineWaves * O::EPW;
+  int node[NP], row[NP], rowNext[NP];
+  double2 xy[NP], uv[NP];
+  load_ids(wave * O::EPW, node, row);
+  load_nodes(node, xy, uv);
+  load_ids(wave * O::EPW + STEP, node, rowNext);
+  for (int v = wave * O::EPW; v < d.ne; v += STEP) {
+    const bool ok = write && v + el < d.ne;
+    double2 xyNext[NP], uvNext[NP], R[NP];
+    int rowAfter[NP];
+    load_nodes(node, xyNext, uvNext);
+    load_ids(v + 2 * STEP, node, rowAfter);
+    line_residual<P, false>(ex, args.basis, mat, line, write, xy, uv, R);
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      if (ok && row[k] != kNoRow) {
+        atomicAdd(&racc[2 * row[k]], R[k].x);
+        atomicAdd(&racc[2 * row[k] + 1], R[k].y);
+      }
+      row[k] = rowNext[k];
+      rowNext[k] = rowAfter[k];
+      xy[k] = xyNext[k];
+      uv[k] = uvNext[k];
+    }
+  }
+  __syncthreads();
+  const gptr_mut<double2> res = gmem_mut(reinterpret_cast<double2 *>(J.residual));
+  for (int i = threadIdx.x; i < d.nr; i += THREADS) {
+    const int node = gmem(J.rows)[d.r0 + i];
+    double2 r = reinterpret_cast<const double2 *>(racc)[i];
+    if (J.accumulate) {
+      const double2 old = res[node];
+      r = make_double2(r.x + old.x, r.y + old.y);
+    }
+    res[node] = r;
+  }
+}
+
 // Per-part kernel of a single job (deterministic plans and parts that take several batches per
 // wavefront): one workgroup per part.
 template <int P, typename T, int WAVES, int MAXB, int MAXR, bool RES, bool JAC, bool DET>
@@ -1971,30 +2216,49 @@ int timed(hipStream_t stream, double *elapsedSeconds, Fn launch) {
 
 constexpr int elem_waves(int order) { return order <= 2 ? 4 : 2; }
 
-template <int P, typename T, bool RES, bool JAC, bool ATOMIC>
+template <int P, typename T, bool RES, bool ATOMIC>
 void launch_element(const ElemArgs &a, hipStream_t stream) {
   constexpr int W = elem_waves(P);
   constexpr int per = W * Ord<P>::EPW;
   const int grid = (a.count + per - 1) / per;
-  if (grid > 0) element_kernel<P, T, W, RES, JAC, ATOMIC><<<grid, W * 64, 0, stream>>>(a);
+  if (grid > 0) element_kernel<P, T, W, RES, ATOMIC><<<grid, W * 64, 0, stream>>>(a);
 }
 
-template <int P, bool RES, bool JAC, bool ATOMIC>
+template <int P, bool RES, bool ATOMIC>
 void launch_element_prec(const ElemArgs &a, int precision, hipStream_t stream) {
   if (precision == FEM_PREC_MIXED) {
-    launch_element<P, float, RES, JAC, ATOMIC>(a, stream);
+    launch_element<P, float, RES, ATOMIC>(a, stream);
   } else {
-    launch_element<P, double, RES, JAC, ATOMIC>(a, stream);
+    launch_element<P, double, RES, ATOMIC>(a, stream);
   }
 }
 
-template <bool RES, bool JAC, bool ATOMIC>
+// Jacobian, with the residual (RES) or without.
+template <bool RES, bool ATOMIC>
 void launch_element_order(int order, const ElemArgs &a, int precision, hipStream_t stream) {
   switch (order) {
-    case 1: launch_element_prec<1, RES, JAC, ATOMIC>(a, precision, stream); break;
-    case 2: launch_element_prec<2, RES, JAC, ATOMIC>(a, precision, stream); break;
-    case 3: launch_element_prec<3, RES, JAC, ATOMIC>(a, precision, stream); break;
-    default: launch_element_prec<4, RES, JAC, ATOMIC>(a, precision, stream); break;
+    case 1: launch_element_prec<1, RES, ATOMIC>(a, precision, stream); break;
+    case 2: launch_element_prec<2, RES, ATOMIC>(a, precision, stream); break;
+    case 3: launch_element_prec<3, RES, ATOMIC>(a, precision, stream); break;
+    default: launch_element_prec<4, RES, ATOMIC>(a, precision, stream); break;
+  }
+}
+
+// Residual alone (FP64 in both precision modes).
+template <int P, bool NL>
+void launch_residual(const ElemArgs &a, hipStream_t stream) {
+  constexpr int per = kLineWaves * LineOrd<P>::EPW;
+  const int grid = (a.count + per - 1) / per;
+  if (grid > 0) residual_kernel<P, NL><<<grid, kLineWaves * 64, 0, stream>>>(a);
+}
+
+template <bool NL>
+void launch_residual_order(int order, const ElemArgs &a, hipStream_t stream) {
+  switch (order) {
+    case 1: launch_residual<1, NL>(a, stream); break;
+    case 2: launch_residual<2, NL>(a, stream); break;
+    case 3: launch_residual<3, NL>(a, stream); break;
+    default: launch_residual<4, NL>(a, stream); break;
   }
 }
 
@@ -2104,21 +2368,21 @@ void launch_split(const SplitJob &job, const Basis1D &basis, int precision, int 
   }
 }
 
-template <int P, bool RES, bool JAC>
+template <int P, bool RES>
 void launch_element_nl(const ElemArgs &a, hipStream_t stream) {
   constexpr int W = elem_waves(P);
   constexpr int per = W * Ord<P>::EPW;
   const int grid = (a.count + per - 1) / per;
-  if (grid > 0) element_kernel_nl<P, W, RES, JAC><<<grid, W * 64, 0, stream>>>(a);
+  if (grid > 0) element_kernel_nl<P, W, RES><<<grid, W * 64, 0, stream>>>(a);
 }
 
-template <bool RES, bool JAC>
+template <bool RES>
 void launch_element_nl_order(int order, const ElemArgs &a, hipStream_t stream) {
   switch (order) {
-    case 1: launch_element_nl<1, RES, JAC>(a, stream); break;
-    case 2: launch_element_nl<2, RES, JAC>(a, stream); break;
-    case 3: launch_element_nl<3, RES, JAC>(a, stream); break;
-    default: launch_element_nl<4, RES, JAC>(a, stream); break;
+    case 1: launch_element_nl<1, RES>(a, stream); break;
+    case 2: launch_element_nl<2, RES>(a, stream); break;
+    case 3: launch_element_nl<3, RES>(a, stream); break;
+    default: launch_element_nl<4, RES>(a, stream); break;
   }
 }
 
@@ -2129,6 +2393,7 @@ struct OwnerLaunch {
   bool det;         // deterministic (colour-phased) sums: per-part kernel
   bool res, jac;    // outputs
   bool rOnlyParts;  // parts sized for residual-only assembly
+  int maxPartRows;  // of a residual-only plan
   bool stream;      // every part is one batch per wavefront: streaming kernel
   int streamGrid;   // persistent workgroups (2 per CU, multiple of 8)
 };
@@ -2158,7 +2423,16 @@ void launch_owner_mode(const OwnerLaunch &L, hipStream_t stream) {
   } else if (L.jac) {
     launch_owner<P, T, cfg.maxRows, false, true, DET>(L, stream);
   } else if (L.rOnlyParts) {
-    launch_owner<P, T, kResidualOnlyMaxRows, true, false, DET>(L, stream);
+    if constexpr (DET) {
+      launch_owner<P, T, kResidualOnlyMaxRows, true, false, true>(L, stream);
+    } else {
+      const int grid = (L.args.totalParts + 7) / 8 * 8;
+      if (L.maxPartRows <= residual_rows(P)) {
+        residual_part_kernel<P, residual_rows(P)><<<grid, kLineWaves * 64, 0, stream>>>(L.args);
+      } else {
+        residual_part_kernel<P, kResidualOnlyMaxRows><<<grid, kLineWaves * 64, 0, stream>>>(L.args);
+      }
+    }
   } else {
     // Residual from a plan whose parts were sized for the Jacobian: rows fit the smaller bound.
     launch_owner<P, T, cfg.maxRows, true, false, DET>(L, stream);
@@ -2236,6 +2510,7 @@ MeshJob make_job(const fem_plan *p, const double *states, const double *coords, 
   MeshJob j{};
   j.visitConn = p->dVisitConn;
   j.visitEid = p->dVisitEid;
+  j.visitRow = p->dVisitRow;
   j.nodeLrow = p->dNodeLrow;
   j.rows = p->dRows;
   j.rowLbase = p->dRowLbase;
@@ -2285,7 +2560,7 @@ int alloc_doubles(int64_t n, double **d, int64_t &bytes) {
 }
 
 void free_plan_arrays(fem_plan *p) {
-  void *ptrs[] = {p->dVisitConn, p->dVisitEid, p->dNodeLrow, p->dRows,  p->dRowLbase, p->dRuns,  p->dColourOff,
+  void *ptrs[] = {p->dVisitConn, p->dVisitEid, p->dVisitRow, p->dNodeLrow, p->dRows,  p->dRowLbase, p->dRuns,  p->dColourOff,
                   p->dPartDesc,  p->dRank,     p->dJob,      p->dJobStart, p->dConn,   p->dCode,  p->dRcode,
                   p->dGline,     p->dGptr,     p->dGsrc,     p->dRline,  p->dRptr,     p->dRsrc,  p->dStage,
                   p->dRstage};
@@ -2319,7 +2594,7 @@ int fem_residual(int order, const int *connPtr, const int *conn, int numElements
   if ((rc = make_basis(order, a.basis)) || (rc = make_material(E, nu, t, a.mat))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return timed(s, elapsedSeconds, [&]() {
-    launch_element_order<true, false, true>(order, a, precision, s);
+    launch_residual_order<false>(order, a, s);
     return FEM_OK;
   });
 }
@@ -2346,8 +2621,8 @@ int fem_jacobian(int order, const int *connPtr, const int *conn, int numElements
   if ((rc = make_basis(order, a.basis)) || (rc = make_material(E, nu, t, a.mat))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return timed(s, elapsedSeconds, [&]() {
-    if (residual) launch_element_order<true, true, true>(order, a, precision, s);
-    else launch_element_order<false, true, true>(order, a, precision, s);
+    if (residual) launch_element_order<true, true>(order, a, precision, s);
+    else launch_element_order<false, true>(order, a, precision, s);
     return FEM_OK;
   });
 }
@@ -2369,7 +2644,7 @@ int fem_residual_nonlinear(int order, const int *connPtr, const int *conn, int n
   if ((rc = make_basis(order, a.basis)) || (rc = make_material(E, nu, t, a.mat))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return timed(s, elapsedSeconds, [&]() {
-    launch_element_nl_order<true, false>(order, a, s);
+    launch_residual_order<true>(order, a, s);
     return FEM_OK;
   });
 }
@@ -2395,8 +2670,8 @@ int fem_jacobian_nonlinear(int order, const int *connPtr, const int *conn, int n
   if ((rc = make_basis(order, a.basis)) || (rc = make_material(E, nu, t, a.mat))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return timed(s, elapsedSeconds, [&]() {
-    if (residual) launch_element_nl_order<true, true>(order, a, s);
-    else launch_element_nl_order<false, true>(order, a, s);
+    if (residual) launch_element_nl_order<true>(order, a, s);
+    else launch_element_nl_order<false>(order, a, s);
     return FEM_OK;
   });
 }
@@ -2434,8 +2709,8 @@ int fem_jacobian_coloured(int order, const int *connPtr, const int *conn, int nu
       a.elemList = colourElements + colourPtr[c];
       a.first = 0;
       a.count = colourPtr[c + 1] - colourPtr[c];
-      if (residual) launch_element_order<true, true, false>(order, a, precision, s);
-      else launch_element_order<false, true, false>(order, a, precision, s);
+      if (residual) launch_element_order<true, false>(order, a, precision, s);
+      else launch_element_order<false, false>(order, a, precision, s);
     }
     return FEM_OK;
   });
@@ -2462,11 +2737,13 @@ int create_plan(int order, int numNodes, int numElements, const int *connPtr, co
   p->numBlocks = h.numBlocks;
   p->elementVisits = int64_t(h.visitEid.size());
   p->maxPartVisits = h.maxPartVisits;
+  p->maxPartRows = h.maxPartRows;
   (void)hipGetDevice(&p->device);
   if (hipDeviceGetAttribute(&p->numCUs, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess) p->numCUs = 0;
   const std::vector<int> jobStart = {0, h.numParts};
   int64_t bytes = 0;
   if ((rc = upload(h.visitConn, &p->dVisitConn, bytes)) || (rc = upload(h.visitEid, &p->dVisitEid, bytes)) ||
+      (rc = upload(h.visitRow, &p->dVisitRow, bytes)) ||
       (rc = upload(h.nodeLrow, &p->dNodeLrow, bytes)) || (rc = upload(h.rows, &p->dRows, bytes)) ||
       (rc = upload(h.rowLbase, &p->dRowLbase, bytes)) || (rc = upload(h.runs, &p->dRuns, bytes)) ||
       (rc = upload(h.colourOff, &p->dColourOff, bytes)) || (rc = upload(h.partDesc, &p->dPartDesc, bytes)) ||
@@ -2699,6 +2976,7 @@ int fem::plan_assemble(fem_plan *plan, const double *states, const double *nodeC
   L.res = residual != nullptr;
   L.jac = matEntries != nullptr;
   L.rOnlyParts = rOnly;
+  L.maxPartRows = plan->maxPartRows;
   L.stream = plan_streams(plan);
   L.streamGrid = stream_grid(plan->numCUs);
   if (plan->dConn && matEntries) {

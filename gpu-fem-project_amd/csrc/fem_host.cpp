@@ -267,7 +267,15 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
   const double scale = std::min(1.0, std::max(partScale, 0.01));
   const int maxVisits = residualOnly ? (1 << 30) : std::max(1, int(cfg.maxVisits * scale));
   const int blockBudget = residualOnly ? maxBlocks : std::max(out.maxRowLength, int(maxBlocks * scale));
-  const int rowBudget = residualOnly ? maxRows : std::max(1, int(maxRows * scale));
+  // Residual-only plans of the line kernel are cut smaller (rowBudget) than their parts may become when nodes of no
+  // element join them (joinBudget); where those do not fit, everything is cut at the largest size.
+  const bool linePlan = residualOnly && !(flags & FEM_PLAN_DETERMINISTIC);
+  int rowBudget = residualOnly ? maxRows : std::max(1, int(maxRows * scale));
+  int joinBudget = rowBudget;
+  if (linePlan) {
+    joinBudget = residual_rows(order);
+    rowBudget = std::min(joinBudget, std::max(128, numNodes / 256));
+  }
   std::vector<int> nptr, nadj;
   node_element_adjacency(numNodes, numElements, N, connPtr, conn, nptr, nadj);
   // Nodes that belong to no element keep zero blocks and zero residual entries. The cut runs over the other
@@ -281,8 +289,12 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
     order_nodes.swap(kept);
   }
   const int numCut = int(order_nodes.size());
-  std::vector<int> cutPtr{0}, partRowCount, partBlockCount;
-  {
+  std::vector<int> cutPtr, partRowCount, partBlockCount;
+  std::vector<std::vector<int>> joined;
+  for (;;) {
+    cutPtr.assign(1, 0);
+    partRowCount.clear();
+    partBlockCount.clear();
     std::vector<int> stamp(numElements, -1);
     int blocks = 0, rowsInPart = 0, visits = 0, part = 0;
     for (int k = 0; k < numCut; k++) {
@@ -309,22 +321,29 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
     cutPtr.push_back(numCut);
     partRowCount.push_back(rowsInPart);
     partBlockCount.push_back(blocks);
-  }
-  {
     const int cutParts = int(cutPtr.size()) - 1;
-    std::vector<std::vector<int>> joined(static_cast<size_t>(cutParts));
-    int p = 0;
+    joined.assign(static_cast<size_t>(cutParts), {});
+    int p = 0, unplaced = -1;
     for (int n : isolated) {
       const int len = rowp[n + 1] - rowp[n];
-      while (p < cutParts && (partRowCount[p] + 1 > rowBudget || partBlockCount[p] + len > blockBudget)) p++;
+      while (p < cutParts && (partRowCount[p] + 1 > joinBudget || partBlockCount[p] + len > blockBudget)) p++;
       if (p == cutParts) {
-        return set_error(FEM_ERR_UNSUPPORTED, "no part has room for the row of node %d, which belongs to no element",
-                         n);
+        unplaced = n;
+        break;
       }
       joined[size_t(p)].push_back(n);
       partRowCount[p]++;
       partBlockCount[p] += len;
     }
+    if (unplaced < 0) break;
+    if (!linePlan || rowBudget == maxRows) {
+      return set_error(FEM_ERR_UNSUPPORTED, "no part has room for the row of node %d, which belongs to no element",
+                       unplaced);
+    }
+    rowBudget = joinBudget = maxRows;
+  }
+  {
+    const int cutParts = int(cutPtr.size()) - 1;
     std::vector<int> placed;
     placed.reserve(size_t(numNodes));
     out.partRowPtr.assign(1, 0);
@@ -351,6 +370,7 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
       base += rowp[n + 1] - rowp[n];
     }
     out.partBlocks[p] = base;
+    out.maxPartRows = std::max(out.maxPartRows, out.partRowPtr[p + 1] - out.partRowPtr[p]);
   }
   // Runs of consecutive node ids: contiguous in both LDS and the BSR value array.
   out.partRunPtr.push_back(0);
@@ -428,6 +448,19 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
       std::memcpy(&out.visitConn[size_t(v) * N], conn + connPtr[out.visitEid[size_t(v)]], N * sizeof(int));
     }
   });
+  if (residualOnly) {  // the part-local row of each visit's nodes, for the line kernel
+    out.visitRow.resize(visits * N);
+    parallel_for(P, [&](int64_t b, int64_t e) {
+      for (int64_t p = b; p < e; p++) {
+        const int *rows = &out.rows[size_t(out.partRowPtr[p])];
+        const int nr = out.partRowPtr[p + 1] - out.partRowPtr[p];
+        for (size_t k = size_t(out.partElemPtr[p]) * N; k < size_t(out.partElemPtr[p + 1]) * N; k++) {
+          const int n = out.visitConn[k], l = out.nodeLrow[size_t(n)];
+          out.visitRow[k] = l < nr && rows[l] == n ? uint16_t(l) : uint16_t(kNoRow);
+        }
+      }
+    });
+  }
   return FEM_OK;
 }
 

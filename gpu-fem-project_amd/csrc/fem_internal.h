@@ -38,8 +38,15 @@ constexpr OwnerConfig owner_config(int order) {
          : order == 3 ? OwnerConfig{4, 1312, 96, 16}
                       : OwnerConfig{4, 1312, 64, 8};
 }
-// Residual-only parts: only the per-row residual lives in LDS.
+// Residual-only parts: only the per-row residual lives in LDS. Deterministic plans take up to kResidualOnlyMaxRows
+// rows per part; the others (line kernel) residual_rows(order): larger parts visit fewer elements twice, smaller
+// ones fill the chip better (701 x 699 elements, us at 1024 / 768 / 512 / 320 rows: order 1 23.2 / 24.0 / 22.3 /
+// 21.7, order 2 56.8 / 54.6 / 53.8 / 58.7, order 3 150 / 130 / 143 / 166, order 4 335 / 376 / 472 / 482). Meshes
+// too small for a part per CU take smaller parts, down to 128 rows (30 x 33, order 4: 17.0 us at 1024 rows, 10.8
+// at 320).
 constexpr int kResidualOnlyMaxRows = 1024;
+constexpr int residual_rows(int order) { return order <= 2 ? 512 : order == 3 ? 768 : kResidualOnlyMaxRows; }
+constexpr int kNoRow = 0xffff;  // PlanHost::visitRow of a node another part owns
 
 // Host-side result of partitioning a mesh into owner parts.
 struct PlanHost {
@@ -52,6 +59,7 @@ struct PlanHost {
   int64_t numBlocks = 0;
   std::vector<int> visitConn;     // [visits*N] nodes of each element visit (parts' visits contiguous)
   std::vector<int> visitEid;      // [visits] element id of each visit
+  std::vector<uint16_t> visitRow; // [visits*N] residual-only plans: the node's row within the part, or kNoRow
   std::vector<int> nodeLrow;      // [numNodes] index of the node within its part's row list
   std::vector<int> partRowPtr;    // [P+1]
   std::vector<int> rows;          // global row (node) ids, ascending within a part
@@ -63,7 +71,7 @@ struct PlanHost {
   std::vector<int> colourOff;     // [P*(C+1)] offsets of each colour within a part's visit list
   std::vector<uint8_t> rank;      // [E][N][rank_pad] rank[e][j][i]: slot of column conn[e,j] in row conn[e,i]
   std::vector<int> partDesc;      // [P*8] (first row, rows, blocks, first run, runs, first visit, visits, 0)
-  int maxPartVisits = 0;
+  int maxPartVisits = 0, maxPartRows = 0;
 };
 
 // Element-once tables (orders 3-4). Every output (a BSR block, or a node's residual pair) is either
@@ -141,6 +149,7 @@ struct fem_plan {
   int64_t deviceBytes = 0;
   int *dVisitConn = nullptr;
   int *dVisitEid = nullptr;
+  uint16_t *dVisitRow = nullptr;
   int *dNodeLrow = nullptr;
   int *dRows = nullptr;
   int *dRowLbase = nullptr;
@@ -166,6 +175,6 @@ struct fem_plan {
   void *dJob = nullptr;      // device job record of the last assembly
   alignas(8) unsigned char hostJob[256] = {};  // host copy of that record
   bool jobUploaded = false;
-  int maxPartVisits = 0;
+  int maxPartVisits = 0, maxPartRows = 0;
   int numCUs = 0;
 };

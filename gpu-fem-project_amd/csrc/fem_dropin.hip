@@ -298,6 +298,7 @@ int fem_jacobian_dropin(int order, const int *connPtr, const int *conn, int numE
 int fem_dropin_cache_clear(void) {
   std::lock_guard<std::mutex> lk(cacheMu);
   cache.clear();
+  pattern_scratch_clear();
   return FEM_OK;
 }
 

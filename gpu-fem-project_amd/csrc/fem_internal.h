@@ -116,6 +116,9 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
                     const int *rowp, const int *cols, const double *nodeCoords, int flags, PlanHost &out,
                     double partScale = 1.0);
 
+// Frees the idle scratch that the device pattern and map builders keep (fem_pattern.hip); returns the blocks freed.
+int pattern_scratch_clear();
+
 // Batches (fem_device.hip). Doubles of element-once staging a Jacobian job of `plan` takes (0: the plan has no
 // element-once tables); fem_batch_add with that staging owned by the caller (`stage`, NULL: the batch's own
 // arena, grown at assembly); whether a plan's parts fit the streaming kernel (graph batches need it).

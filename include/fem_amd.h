@@ -144,8 +144,9 @@ int fem_write_bdf(const char *path, int order, int numNodes, int numElements, co
  * The same pattern and map as fem_bsr_pattern_rowp/_cols and fem_element_bcsr_map (identical arrays), built
  * on the GPU from device arrays, in work ordered on `stream` (a hipStream_t; NULL = default stream). These
  * replace the host set-up the reference leaves to TACS (createSchurMat, verification/TestKernels.cpp:105)
- * and generateElementBCSRMap (verification/TACSHelpers.h:138-182). Each call allocates and frees its own
- * scratch and returns after its work has finished. connPtr entries must index valid conn entries, as for
+ * and generateElementBCSRMap (verification/TACSHelpers.h:138-182). Each call returns after its work has
+ * finished. Scratch comes from one block per GPU that the library keeps (up to 256 MiB, released by
+ * fem_dropin_cache_clear); calls that overlap, and larger meshes, allocate and free their own. connPtr entries must index valid conn entries, as for
  * every entry point here.
  * fem_bsr_pattern_device fills rowp (numNodes + 1 entries) and *numBlocks. Pass cols = NULL to size the
  * pattern, then call again with cols of colsCapacity >= *numBlocks entries. FEM_ERR_UNSUPPORTED if a node's
@@ -195,6 +196,7 @@ int fem_jacobian(int order, const int *connPtr, const int *conn, int numElements
 int fem_jacobian_dropin(int order, const int *connPtr, const int *conn, int numElements, const double *states,
                         const double *nodeCoords, double E, double nu, double t, const int *elementBCSRMap,
                         double *residual, double *matEntries, int precision, void *stream, double *elapsedSeconds);
+/* Releases the cached plans and the pattern builders' idle scratch. */
 int fem_dropin_cache_clear(void);
 /* Whether the combination is cached (*cached) and served by a plan (*usesPlan; else by fem_jacobian). */
 int fem_dropin_cache_info(int order, const int *connPtr, const int *conn, int numElements, const int *elementBCSRMap,

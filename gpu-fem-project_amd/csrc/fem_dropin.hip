@@ -5,11 +5,11 @@
 // every element contribution into matEntries with atomics (fem_jacobian does the same here). This entry point
 // builds, on first use of a (connPtr, conn, map, numElements, order) combination, the BSR pattern and element map
 // of the connectivity on the device; if that map equals the caller's, the caller's matrix has this library's
-// pattern, and a resident plan is built and cached. Calls then run the plan's kernels in accumulate mode (orders
-// 1-2: owner-computes parts; 3-4: element-once traversal and gathers): every output is read and written once
-// (+=, the reference's semantics), with no atomics. Every call first checks that the cached arrays are unchanged (a 64-bit checksum of conn and of
-// a strided sample of the map); a change rebuilds the entry. Anything else (orders 3-4, a different pattern, a failed
-// build) runs fem_jacobian.
+// pattern, and a resident plan is built and cached. Calls then run the plan's kernels in accumulate mode
+// (owner-computes parts): every output is read and written once (+=, the reference's semantics), with no atomics.
+// Every call first checks that the cached arrays are unchanged (a 64-bit checksum of conn and of a strided sample of
+// the map); a change rebuilds the entry. Anything else (orders 3-4, a different pattern, a failed build) runs
+// fem_jacobian.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,6 +36,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int64_t kMapStride = 61;  // map entries sampled by the per-call check
 constexpr size_t kMaxEntries = 4;   // cached plans (least recently used evicted)
+constexpr int kCheckBlocks = 1024;  // most workgroups of a check: four per CU
 
 // 32-bit finaliser of a (position, value) pair (MurmurHash3's fmix32 on a multiplicative combination).
 __device__ __forceinline__ unsigned int mix32(unsigned int k, unsigned int v) {
@@ -47,26 +48,53 @@ __device__ __forceinline__ unsigned int mix32(unsigned int k, unsigned int v) {
   return x ^ (x >> 16);
 }
 
+// What one workgroup of the check saw: its share of the sum, the largest node id (-1: none) and whether an id is negative.
+struct Partial {
+  unsigned long long sum;
+  int maxNode, negative;
+};
+
 // Order-independent 64-bit sum of mix32 over conn[connPtr[e] + a] (all e, a) and map[k * stride] (sampled), plus
-// the largest node id and a flag for a negative one. One atomic of each kind per workgroup.
+// the largest node id and a flag for a negative one: one Partial per workgroup, in host memory, which the host adds up
+// after it has waited for the stream. Bound by latency (two dependent loads a reference, a line of the map a
+// sample), so a thread has kBatch references on their way at a time, and NPE is a constant for the division. One
+// atomic of each kind per workgroup and one load in flight took 31 us at 122 850 quadratic elements, with the copies
+// that cleared and fetched the results 85 us of a call's 319; now 11 us (batches of four on 512 workgroups: 13) and 14
+// of 248.
+constexpr int kBatch = 2;
+template <int NPE>
 __global__ __launch_bounds__(kThreads) void checksum_kernel(const int *connPtr, const int *conn, int numElements,
-                                                            int npe, const int *map, int64_t mapSamples,
-                                                            unsigned long long *sum, int *maxNode, int *negative) {
-  const int64_t refs = int64_t(numElements) * npe;
+                                                            const int *map, int64_t mapSamples, Partial *out) {
+  const int64_t refs = int64_t(numElements) * NPE;
+  const int64_t first = int64_t(blockIdx.x) * kThreads + threadIdx.x, step = int64_t(gridDim.x) * kThreads;
   unsigned long long h = 0;
   int mx = -1;
   bool neg = false;
-  for (int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x; k < refs + mapSamples;
-       k += int64_t(gridDim.x) * kThreads) {
-    if (k < refs) {
-      const int e = int(k / npe), a = int(k - int64_t(e) * npe);
-      const int n = conn[int64_t(connPtr[e]) + a];
-      h += mix32(unsigned(k), unsigned(n));
-      mx = max(mx, n);
-      neg = neg || n < 0;
-    } else {
-      const int64_t s = k - refs;
-      h += (unsigned long long)mix32(unsigned(s) ^ 0x5bd1e995u, unsigned(map[s * kMapStride])) << 20;
+  for (int64_t s0 = first; s0 < mapSamples; s0 += kBatch * step) {
+    int v[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; i++) v[i] = s0 + i * step < mapSamples ? map[(s0 + i * step) * kMapStride] : 0;
+#pragma unroll
+    for (int i = 0; i < kBatch; i++) {
+      const int64_t s = s0 + i * step;
+      if (s < mapSamples) h += (unsigned long long)mix32(unsigned(s) ^ 0x5bd1e995u, unsigned(v[i])) << 20;
+    }
+  }
+  for (int64_t k0 = first; k0 < refs; k0 += kBatch * step) {
+    int at[kBatch], n[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; i++) at[i] = k0 + i * step < refs ? connPtr[(k0 + i * step) / NPE] : 0;
+#pragma unroll
+    for (int i = 0; i < kBatch; i++)
+      n[i] = k0 + i * step < refs ? conn[int64_t(at[i]) + int((k0 + i * step) % NPE)] : 0;
+#pragma unroll
+    for (int i = 0; i < kBatch; i++) {
+      const int64_t k = k0 + i * step;
+      if (k < refs) {
+        h += mix32(unsigned(k), unsigned(n[i]));
+        mx = max(mx, n[i]);
+        neg = neg || n[i] < 0;
+      }
     }
   }
   __shared__ unsigned long long hs[kThreads / 64];
@@ -84,16 +112,13 @@ __global__ __launch_bounds__(kThreads) void checksum_kernel(const int *connPtr, 
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long bh = 0;
-    int bm = -1, bn = 0;
+    Partial p{0, -1, 0};
     for (int i = 0; i < kThreads / 64; i++) {
-      bh += hs[i];
-      bm = max(bm, ms[i]);
-      bn |= ns[i];
+      p.sum += hs[i];
+      p.maxNode = max(p.maxNode, ms[i]);
+      p.negative |= ns[i];
     }
-    atomicAdd(sum, bh);
-    atomicMax(maxNode, bm);
-    if (bn) atomicOr(negative, 1);
+    out[blockIdx.x] = p;
   }
 }
 
@@ -110,12 +135,10 @@ struct Entry {
   unsigned long long sum = 0;
   fem_plan *plan = nullptr;  // NULL: this combination runs fem_jacobian
   uint64_t lastUse = 0;
-  unsigned long long *dSum = nullptr;  // the check's device results: checksum, then (largest node, negative)
-  int *dInts = nullptr;
+  Partial *partial = nullptr;  // [kCheckBlocks] the check's results, host memory that the device writes
   ~Entry() {
     fem_plan_destroy(plan);
-    if (dSum) (void)hipFree(dSum);
-    if (dInts) (void)hipFree(dInts);
+    if (partial) (void)hipHostFree(partial);
   }
 };
 
@@ -148,30 +171,28 @@ int64_t map_samples(int numElements, int npe) {
   return (n + kMapStride - 1) / kMapStride;
 }
 
-// Checksum (and largest node id, negative-id flag) of the entry's arrays, in the entry's device results;
-// synchronises `stream`.
+// Checksum (and largest node id, negative-id flag) of the entry's arrays; synchronises `stream`.
 int checksum(Entry &e, hipStream_t stream, unsigned long long &sum, int &maxNode, bool &negative) {
-  const int order = e.order, numElements = e.numElements;
-  const int *connPtr = e.connPtr, *conn = e.conn, *map = e.map;
-  const int npe = nodes_per_element(order);
-  if (!e.dSum) FEM_DI_CHECK(hipMalloc(reinterpret_cast<void **>(&e.dSum), sizeof(unsigned long long)));
-  if (!e.dInts) FEM_DI_CHECK(hipMalloc(reinterpret_cast<void **>(&e.dInts), 2 * sizeof(int)));
-  unsigned long long *dSum = e.dSum;
-  int *dInts = e.dInts;
-  const int init[2] = {-1, 0};
-  const unsigned long long zero = 0;
-  FEM_DI_CHECK(hipMemcpyAsync(dSum, &zero, sizeof(zero), hipMemcpyHostToDevice, stream));
-  FEM_DI_CHECK(hipMemcpyAsync(dInts, init, sizeof(init), hipMemcpyHostToDevice, stream));
-  const int64_t work = int64_t(numElements) * npe + map_samples(numElements, npe);
-  checksum_kernel<<<grid_for(work), kThreads, 0, stream>>>(connPtr, conn, numElements, npe, map,
-                                                          map_samples(numElements, npe), dSum, dInts, dInts + 1);
+  const int npe = nodes_per_element(e.order);
+  if (!e.partial)
+    FEM_DI_CHECK(hipHostMalloc(reinterpret_cast<void **>(&e.partial), kCheckBlocks * sizeof(Partial), hipHostMallocDefault));
+  const int64_t samples = map_samples(e.numElements, npe), work = int64_t(e.numElements) * npe;
+  const int64_t blocks = (work + kThreads * kBatch - 1) / (kThreads * kBatch);
+  const unsigned grid = unsigned(std::clamp<int64_t>(blocks, 1, kCheckBlocks));
+  if (npe == 4)
+    checksum_kernel<4><<<grid, kThreads, 0, stream>>>(e.connPtr, e.conn, e.numElements, e.map, samples, e.partial);
+  else
+    checksum_kernel<9><<<grid, kThreads, 0, stream>>>(e.connPtr, e.conn, e.numElements, e.map, samples, e.partial);
   FEM_DI_CHECK(hipGetLastError());
-  int h[2];
-  FEM_DI_CHECK(hipMemcpyAsync(&sum, dSum, sizeof(sum), hipMemcpyDeviceToHost, stream));
-  FEM_DI_CHECK(hipMemcpyAsync(h, dInts, sizeof(h), hipMemcpyDeviceToHost, stream));
   FEM_DI_CHECK(hipStreamSynchronize(stream));
-  maxNode = h[0];
-  negative = h[1] != 0;
+  sum = 0;
+  maxNode = -1;
+  negative = false;
+  for (unsigned i = 0; i < grid; i++) {
+    sum += e.partial[i].sum;
+    maxNode = std::max(maxNode, e.partial[i].maxNode);
+    negative = negative || e.partial[i].negative;
+  }
   return FEM_OK;
 }
 

@@ -855,7 +855,7 @@ __device__ __forceinline__ int find_job(const int *start, int n, int64_t x) {
 }
 
 // A batch's element-once jobs of one order: counts = (jobs, units, staged blocks, staged residual entries)
-// in device memory (so a recorded graph replays any batch), unitStart[j] the first unit of job j, a unit
+// in device memory, unitStart[j] the first unit of job j, a unit
 // being WAVES * EPW elements. Persistent: workgroups stride over the units.
 template <int P, typename T, int WAVES, bool RES>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(3)))
@@ -1299,7 +1299,6 @@ struct MeshJob {
 struct OwnerArgs {
   const MeshJob *jobs;    // device job table
   const int *jobStart;    // [numJobs+1] first global part of each job
-  const int *counts;      // if non-NULL: device (numJobs, totalParts), read instead of the two fields below
   int numJobs;
   int totalParts;
   Basis1D basis;
@@ -2122,8 +2121,8 @@ void owner_stream_kernel(const OwnerArgs args) {
   // Contiguous range of global parts per workgroup; workgroup w runs on XCD w % 8, and each XCD's
   // workgroups share one contiguous (spatially adjacent, Morton-ordered) stretch of parts.
   const int xcd = int(blockIdx.x % 8), slot = int(blockIdx.x / 8), perX = int(gridDim.x / 8);
-  const int numJobs = uniform(args.counts ? args.counts[0] : args.numJobs);
-  const int64_t np = uniform(args.counts ? args.counts[1] : args.totalParts);
+  const int numJobs = args.numJobs;
+  const int64_t np = args.totalParts;
   const int xb = int(np * xcd / 8), xe = int(np * (xcd + 1) / 8);
   const int pb = xb + int(int64_t(xe - xb) * slot / perX);
   const int pe = xb + int(int64_t(xe - xb) * (slot + 1) / perX);
@@ -2333,41 +2332,69 @@ __device__ __forceinline__ void gather_one(const int *line, const int *ptr, cons
   *o = sum;
 }
 
-template <int C>
-__global__ __launch_bounds__(256) void gather_shared(const int *line, const int *ptr, const int *src,
-                                                     const double *stage, double *out, int outputs, int n,
-                                                     int accumulate) {
-  const int64_t total = int64_t(n) * 4, stride = int64_t(gridDim.x) * 256;
-  for (int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x; t < total; t += stride) {
-    gather_one<C>(line, ptr, src, stage, out, outputs, t / 4, int(t % 4), accumulate != 0);
-  }
-}
-
-template <int C>
-void launch_gather_shared(const int *line, const int *ptr, const int *src, const double *stage, double *out,
-                          int outputs, int n, int accumulate, hipStream_t stream) {
-  const int64_t blocks = (int64_t(n) * 4 + 255) / 256;
-  if (n > 0) {
-    gather_shared<C><<<unsigned(std::min<int64_t>(blocks, 1 << 20)), 256, 0, stream>>>(line, ptr, src, stage, out,
-                                                                                        outputs, n, accumulate);
-  }
-}
-
-// The gathers of a batch's element-once jobs: C = 4, the blocks' lines (lineStart[j]: job j's first line over all
-// jobs, counts[2] in total), or C = 2, the residual's (counts[3]; jobs without a residual have none).
-template <int C>
-__global__ __launch_bounds__(256) void gather_batch(const SplitJob *jobs, const int *lineStart, const int *counts) {
-  const int numJobs = counts[0];
-  const int64_t total = int64_t(counts[C == 4 ? 2 : 3]) * 4, stride = int64_t(gridDim.x) * 256;
+// Both gathers of one plan in one launch: the lines of the blocks, then those of the residual (`lines` in total; an
+// order-3 mesh of 22 499 elements, mixed: 26 + 4 us in two launches, 25 in one).
+__global__ __launch_bounds__(256) void gather_shared(const SplitJob job, int64_t lines) {
+  const int64_t total = lines * 4, stride = int64_t(gridDim.x) * 256;
+  const bool accumulate = job.accumulate != 0;
   for (int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x; t < total; t += stride) {
     const int64_t i = t / 4;
-    const int j = find_job(lineStart, numJobs, i), h = int(t % 4);
-    const SplitJob &job = jobs[j];
-    if (C == 4) {
-      gather_one<4>(job.gline, job.gptr, job.gsrc, job.stage, job.values, job.numBlocks, i - lineStart[j], h);
+    const int h = int(t % 4);
+    if (i < job.numGather) {
+      gather_one<4>(job.gline, job.gptr, job.gsrc, job.stage, job.values, job.numBlocks, i, h, accumulate);
     } else {
-      gather_one<2>(job.rline, job.rptr, job.rsrc, job.rstage, job.residual, job.numNodes, i - lineStart[j], h);
+      gather_one<2>(job.rline, job.rptr, job.rsrc, job.rstage, job.residual, job.numNodes, i - job.numGather, h,
+                    accumulate);
     }
+  }
+}
+
+// The gathers of all element-once groups of a batch in one launch, over 2 G segments of lines: segment 2 g holds the
+// block lines of group g's jobs, job j's from start[2 g][j] on, and segment 2 g + 1 the residual's. The wavefronts
+// share the lines of all segments in contiguous runs of steps of 16, so a run lies in few jobs, whose records are
+// looked up once and are scalar. What a wavefront looks up before its first line, one dependent load after another,
+// is what this is bound by, so more workgroups than the chip holds make it slower (24 meshes, 28 286 elements of orders
+// 3-4, mixed: the whole batch 258 us with 8 workgroups per CU, 282 with 4, 273 with 64; one strided launch per group and
+// output, each line's job looked up by its lanes, took 83 us of gathers and two more launches than this one's 62).
+constexpr int kSplitGroups = 4;
+struct BatchGather {
+  const SplitJob *jobs[kSplitGroups];
+  const int *start[2 * kSplitGroups];
+  int numJobs[kSplitGroups];
+  int lines[2 * kSplitGroups];
+};
+
+__global__ __launch_bounds__(256) void gather_batch(const BatchGather b) {
+  const int64_t wave = uniform(int(blockIdx.x * 4 + threadIdx.x / 64)), waves = int64_t(gridDim.x) * 4;
+  const int row = int(threadIdx.x % 64) / 4, h = int(threadIdx.x % 4);
+  int64_t steps = 0;
+#pragma unroll
+  for (int seg = 0; seg < 2 * kSplitGroups; seg++) steps += (b.lines[seg] + 15) / 16;
+  int64_t first = steps * wave / waves, last = steps * (wave + 1) / waves;  // of the steps that are left
+#pragma unroll 1
+  for (int seg = 0; seg < 2 * kSplitGroups && last > 0; seg++) {
+    const int64_t here = (b.lines[seg] + 15) / 16;
+    if (first < here) {
+      const int end = int(min(16 * last, int64_t(b.lines[seg])));
+      int at = int(16 * max(first, int64_t(0)));
+      const int *start = b.start[seg];
+      for (int j = uniform(find_job(start, b.numJobs[seg / 2], at)); at < end; j++) {
+        const SplitJob job = b.jobs[seg / 2][j];
+        const int j0 = start[j], jend = min(start[j + 1], end);
+        for (; at < jend; at += 16) {
+          const int i = at + row;
+          if (i >= jend) continue;
+          if (seg % 2) {
+            gather_one<2>(job.rline, job.rptr, job.rsrc, job.rstage, job.residual, job.numNodes, i - j0, h);
+          } else {
+            gather_one<4>(job.gline, job.gptr, job.gsrc, job.stage, job.values, job.numBlocks, i - j0, h);
+          }
+        }
+        at = jend;
+      }
+    }
+    first -= here;
+    last -= here;
   }
 }
 
@@ -2383,12 +2410,8 @@ void launch_split(const SplitJob &job, const Basis1D &basis, int precision, int 
     if (res) launch_element_split<P, double, true>(job, basis, waves, s);
     else launch_element_split<P, double, false>(job, basis, waves, s);
   }
-  launch_gather_shared<4>(job.gline, job.gptr, job.gsrc, job.stage, job.values, job.numBlocks, job.numGather,
-                          job.accumulate, s);
-  if (res) {
-    launch_gather_shared<2>(job.rline, job.rptr, job.rsrc, job.rstage, job.residual, job.numNodes, job.numRgather,
-                            job.accumulate, s);
-  }
+  const int64_t lines = int64_t(job.numGather) + (res ? job.numRgather : 0), blocks = (4 * lines + 255) / 256;
+  if (lines > 0) gather_shared<<<unsigned(std::min<int64_t>(blocks, 1 << 20)), 256, 0, s>>>(job, lines);
 }
 
 template <int P, bool RES>
@@ -2428,7 +2451,7 @@ void launch_owner(const OwnerLaunch &L, hipStream_t stream) {
     if (L.stream) {
       // streamGrid is two workgroups per CU; 8-wave workgroups fill a CU's LDS alone.
       const int persistent = cfg.waves >= 8 ? std::max(8, L.streamGrid / 16 * 8) : L.streamGrid;
-      const int grid = std::min(persistent, ((L.args.totalParts + 7) / 8) * 8);
+      const int grid = std::min(persistent, std::max((L.args.totalParts + 7) / 8, 1) * 8);
       owner_stream_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC><<<grid, cfg.waves * 64, 0, stream>>>(
           L.args);
       return;
@@ -3046,7 +3069,6 @@ struct fem_batch {
     std::vector<int64_t> stageOff, rstageOff;             // each job's staging, in doubles into the arena
   };
   static constexpr int kGroups = 12;
-  static constexpr int kSplitGroups = 4;
   Group groups[kGroups];
   SplitGroup split[kSplitGroups];
   // Staging of the element-once jobs: the batch's own (so that batches holding one plan can run
@@ -3057,7 +3079,7 @@ struct fem_batch {
   int flags = 0;
   int numCUs = 0;
   int numJobs = 0;
-  // One device block at a fixed address (a captured graph refers to it), laid out as
+  // One device block, laid out as
   //   counts [kGroups + kSplitGroups][4] int (owner: numJobs, totalParts; element-once: numJobs, units,
   //     staged blocks, staged residuals)
   //   | jobStart [kGroups][maxJobs + 1] int | jobs [kGroups][maxJobs] MeshJob
@@ -3069,7 +3091,6 @@ struct fem_batch {
   size_t jobStartOffset = 0, jobsOffset = 0, splitStartOffset = 0, splitJobsOffset = 0, tableBytes = 0;
   hipEvent_t staged = nullptr;  // recorded after the copy: the host mirror is rewritten only once it has run
   bool stagedPending = false;
-  hipGraphExec_t graph[2] = {nullptr, nullptr};  // per precision
   // Jobs of deterministic and residual-only plans (batches without graphs only): each runs as its plan's own
   // assembly on the batch's stream, after the groups.
   struct Solo {
@@ -3079,8 +3100,7 @@ struct fem_batch {
     double *residual, *values;
   };
   std::vector<Solo> solo;
-  bool assembled = false;                          // fem_batch_assemble has staged job tables
-  hipStream_t captureStream = nullptr;             // graphs are recorded here and replayed on any stream
+  bool assembled = false;  // fem_batch_assemble has staged job tables
 
   int *dCounts() const { return reinterpret_cast<int *>(dTables); }
   int *dJobStart() const { return reinterpret_cast<int *>(dTables + jobStartOffset); }
@@ -3096,27 +3116,21 @@ struct fem_batch {
 namespace {
 
 void free_batch(fem_batch *b) {
-  for (auto &g : b->graph) {
-    if (g) (void)hipGraphExecDestroy(g);
-    g = nullptr;
-  }
   if (b->staged) {
     if (b->stagedPending) (void)hipEventSynchronize(b->staged);
     (void)hipEventDestroy(b->staged);
   }
-  if (b->captureStream) (void)hipStreamDestroy(b->captureStream);
   if (b->dArena) (void)hipFree(b->dArena);
   if (b->dTables) (void)hipFree(b->dTables);
   if (b->hTables) (void)hipHostFree(b->hTables);
 }
 
-OwnerLaunch batch_group_launch(const fem_batch *b, int gi, int precision, bool fromDevice) {
+OwnerLaunch batch_group_launch(const fem_batch *b, int gi, int precision) {
   const fem_batch::Group &g = b->groups[gi];
   OwnerLaunch L{};
   make_basis(gi / 3 + 1, L.args.basis);
   L.args.jobs = b->dJobs() + size_t(gi) * b->maxJobs;
   L.args.jobStart = b->dJobStart() + size_t(gi) * (b->maxJobs + 1);
-  L.args.counts = fromDevice ? b->dCounts() + 4 * gi : nullptr;
   L.args.numJobs = int(g.jobs.size());
   L.args.totalParts = g.jobStart.back();
   L.precision = precision;
@@ -3124,80 +3138,76 @@ OwnerLaunch batch_group_launch(const fem_batch *b, int gi, int precision, bool f
   L.res = gi % 3 != 1;
   L.jac = gi % 3 != 0;
   L.rOnlyParts = false;
-  L.stream = fromDevice || (g.stream && b->numCUs > 0);
+  L.stream = g.stream && b->numCUs > 0;
   L.streamGrid = stream_grid(b->numCUs);
   return L;
 }
 
-// Launches of element-once group g (order 3 + g / 2; with residual if g is odd): the tiled kernel over the
-// group's units, then the gathers of its staged blocks and residual entries. The kernels read the group's
-// counts from device memory; `fixedGrid` sizes the grids for any batch (graph recording), otherwise from the
-// host's counts.
+// Launch of element-once group g (order 3 + g / 2; with residual if g is odd): the tiled kernel over the group's
+// units, whose counts it reads from device memory.
 template <int P, typename T, bool RES>
-void launch_split_group_t(const fem_batch *b, int g, bool fixedGrid, hipStream_t s) {
+void launch_split_group_t(const fem_batch *b, int g, hipStream_t s) {
   const fem_batch::SplitGroup &sg = b->split[g];
   const int *counts = b->dCounts() + 4 * (fem_batch::kGroups + g);
   const SplitJob *jobs = reinterpret_cast<const SplitJob *>(b->dTables + b->splitJobsAt(g));
   const int *unitStart = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 0));
-  const int *gStart = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 1));
-  const int *rStart = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 2));
   const int cap = std::max(8 * b->numCUs, 64);
-  auto grid = [&](int64_t work) { return unsigned(fixedGrid ? cap : std::max<int64_t>(1, std::min<int64_t>(work, cap))); };
+  const unsigned grid = unsigned(std::clamp(sg.unitStart.back(), 1, cap));
   Basis1D basis;
   make_basis(P, basis);
-  element_tiled_batch<P, T, kTiledWaves, RES><<<grid(sg.unitStart.back()), kTiledWaves * 64, 0, s>>>(jobs, unitStart,
-                                                                                                   counts, basis);
-  gather_batch<4><<<grid((int64_t(sg.gStart.back()) * 4 + 255) / 256), 256, 0, s>>>(jobs, gStart, counts);
-  if (RES) gather_batch<2><<<grid((int64_t(sg.rStart.back()) * 2 + 255) / 256), 256, 0, s>>>(jobs, rStart, counts);
+  element_tiled_batch<P, T, kTiledWaves, RES><<<grid, kTiledWaves * 64, 0, s>>>(jobs, unitStart, counts, basis);
 }
 
-void launch_split_group(const fem_batch *b, int g, int precision, bool fixedGrid, hipStream_t s) {
+void launch_split_group(const fem_batch *b, int g, int precision, hipStream_t s) {
   const bool mixed = precision == FEM_PREC_MIXED;
   switch (g) {
-    case 0: mixed ? launch_split_group_t<3, float, false>(b, g, fixedGrid, s) : launch_split_group_t<3, double, false>(b, g, fixedGrid, s); break;
-    case 1: mixed ? launch_split_group_t<3, float, true>(b, g, fixedGrid, s) : launch_split_group_t<3, double, true>(b, g, fixedGrid, s); break;
-    case 2: mixed ? launch_split_group_t<4, float, false>(b, g, fixedGrid, s) : launch_split_group_t<4, double, false>(b, g, fixedGrid, s); break;
-    default: mixed ? launch_split_group_t<4, float, true>(b, g, fixedGrid, s) : launch_split_group_t<4, double, true>(b, g, fixedGrid, s); break;
+    case 0: mixed ? launch_split_group_t<3, float, false>(b, g, s) : launch_split_group_t<3, double, false>(b, g, s); break;
+    case 1: mixed ? launch_split_group_t<3, float, true>(b, g, s) : launch_split_group_t<3, double, true>(b, g, s); break;
+    case 2: mixed ? launch_split_group_t<4, float, false>(b, g, s) : launch_split_group_t<4, double, false>(b, g, s); break;
+    default: mixed ? launch_split_group_t<4, float, true>(b, g, s) : launch_split_group_t<4, double, true>(b, g, s); break;
   }
 }
 
-// Graph of the 12 group launches, each reading its job count from device memory (empty groups exit).
-// Recorded on the batch's own stream (capture is not allowed on the null stream); it is replayed on the
-// caller's stream.
-int capture_batch_graph(fem_batch *b, int precision) {
-  if (!b->captureStream) FEM_HIP_CHECK(hipStreamCreateWithFlags(&b->captureStream, hipStreamNonBlocking));
-  hipStream_t s = b->captureStream;
-  hipGraph_t graph = nullptr;
-  FEM_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  for (int gi = 0; gi < fem_batch::kGroups; gi++) {
-    OwnerLaunch L = batch_group_launch(b, gi, precision, true);
-    L.args.totalParts = L.streamGrid;  // host-side grid bound only; the kernel reads the device count
-    launch_owner_any(gi / 3 + 1, L, s);
+// Launch of the gathers of all element-once groups.
+void launch_split_gather(const fem_batch *b, hipStream_t s) {
+  BatchGather args{};
+  int64_t lines = 0;
+  for (int g = 0; g < kSplitGroups; g++) {
+    const fem_batch::SplitGroup &sg = b->split[g];
+    args.jobs[g] = reinterpret_cast<const SplitJob *>(b->dTables + b->splitJobsAt(g));
+    args.numJobs[g] = int(sg.jobs.size());
+    for (int k = 0; k < 2; k++) {
+      args.start[2 * g + k] = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 1 + k));
+      if (k == 0 || g % 2 == 1) args.lines[2 * g + k] = (k ? sg.rStart : sg.gStart).back();
+      lines += args.lines[2 * g + k];
+    }
   }
-  for (int g = 0; g < fem_batch::kSplitGroups; g++) launch_split_group(b, g, precision, true, s);
-  FEM_HIP_CHECK(hipStreamEndCapture(s, &graph));
-  hipError_t e = hipGraphInstantiate(&b->graph[precision], graph, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(graph);
-  if (e != hipSuccess) return set_error(FEM_ERR_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
-  return FEM_OK;
+  const int cap = std::max(8 * b->numCUs, 64);
+  gather_batch<<<unsigned(std::clamp<int64_t>((4 * lines + 255) / 256, 1, cap)), 256, 0, s>>>(args);
 }
 
 }  // namespace
 
-int fem::batch_prepare_graph(fem_batch *b, int precision) {
+int fem::batch_prepare(fem_batch *b, int precision) {
   if (!b) return set_error(FEM_ERR_NULL_POINTER, "batch is NULL");
   if (precision != FEM_PREC_FP64 && precision != FEM_PREC_MIXED) {
     return set_error(FEM_ERR_INVALID_ARGUMENT, "unknown precision mode %d", precision);
   }
-  if (!(b->flags & FEM_BATCH_GRAPH) || b->graph[precision]) return FEM_OK;
-  int rc = capture_batch_graph(b, precision);
-  if (rc) return rc;
-  if (!b->assembled) {
-    // One replay while every job count in the tables is still zero (all kernels exit at once): the runtime's
-    // first-launch allocations (scratch of kernels that spill, graph kernel arguments) happen now, not later.
-    FEM_HIP_CHECK(hipGraphLaunch(b->graph[precision], b->captureStream));
-    FEM_HIP_CHECK(hipStreamSynchronize(b->captureStream));
+  if (!(b->flags & FEM_BATCH_GRAPH) || b->assembled) return FEM_OK;  // until then the device tables are zero
+  hipStream_t s = nullptr;
+  FEM_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+  for (int gi = 0; gi < fem_batch::kGroups; gi++) {
+    OwnerLaunch L = batch_group_launch(b, gi, precision);
+    L.stream = true;
+    launch_owner_any(gi / 3 + 1, L, s);
   }
+  for (int g = 0; g < kSplitGroups; g++) launch_split_group(b, g, precision, s);
+  launch_split_gather(b, s);
+  hipError_t e = hipGetLastError();
+  const hipError_t w = hipStreamSynchronize(s);
+  (void)hipStreamDestroy(s);
+  if (e == hipSuccess) e = w;
+  if (e != hipSuccess) return set_error(FEM_ERR_HIP, "preparing a batch failed: %s", hipGetErrorString(e));
   return FEM_OK;
 }
 
@@ -3212,7 +3222,7 @@ int fem_batch_create(int maxJobs, int flags, fem_batch **batch) {
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&b->numCUs, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) b->numCUs = 0;
-  const size_t G = fem_batch::kGroups, SG = fem_batch::kSplitGroups;
+  const size_t G = fem_batch::kGroups, SG = kSplitGroups;
   b->jobStartOffset = 4 * (G + SG) * sizeof(int);
   b->jobsOffset = (b->jobStartOffset + G * size_t(maxJobs + 1) * sizeof(int) + 255) / 256 * 256;
   b->splitStartOffset = b->jobsOffset + G * size_t(maxJobs) * sizeof(MeshJob);
@@ -3353,7 +3363,6 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
     return set_error(FEM_ERR_INVALID_ARGUMENT, "unknown precision mode %d", precision);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool useGraph = (batch->flags & FEM_BATCH_GRAPH) != 0;
   // The previous call's copy must have run before the pinned mirror is rewritten.
   if (batch->stagedPending) {
     FEM_HIP_CHECK(hipEventSynchronize(batch->staged));
@@ -3403,7 +3412,7 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
                 g.jobStart.size() * sizeof(int));
     copyEnd = batch->jobsOffset + (size_t(gi) * batch->maxJobs + g.jobs.size()) * sizeof(MeshJob);
   }
-  for (int g = 0; g < fem_batch::kSplitGroups; g++) {
+  for (int g = 0; g < kSplitGroups; g++) {
     const fem_batch::SplitGroup &sg = batch->split[g];
     int *cnt = batch->hCounts() + 4 * (fem_batch::kGroups + g);
     cnt[0] = int(sg.jobs.size());
@@ -3422,20 +3431,11 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
   FEM_HIP_CHECK(hipEventRecord(batch->staged, s));
   batch->stagedPending = true;
   batch->assembled = true;
-  if (useGraph && !batch->graph[precision]) {
-    int rc = capture_batch_graph(batch, precision);
-    if (rc) return rc;
-  }
   return timed(s, elapsedSeconds, [&]() -> int {
-    if (useGraph) {
-      hipError_t e = hipGraphLaunch(batch->graph[precision], s);
-      if (e != hipSuccess) return set_error(FEM_ERR_HIP, "hipGraphLaunch failed: %s", hipGetErrorString(e));
-      return FEM_OK;
-    }
     for (int gi = 0; gi < fem_batch::kGroups; gi++) {
       fem_batch::Group &g = batch->groups[gi];
       if (g.jobs.empty()) continue;
-      const OwnerLaunch L = batch_group_launch(batch, gi, precision, false);
+      const OwnerLaunch L = batch_group_launch(batch, gi, precision);
       if (L.stream) {
         launch_owner_any(gi / 3 + 1, L, s);
       } else {
@@ -3449,9 +3449,13 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
         }
       }
     }
-    for (int g = 0; g < fem_batch::kSplitGroups; g++) {
-      if (!batch->split[g].jobs.empty()) launch_split_group(batch, g, precision, false, s);
+    bool staged = false;
+    for (int g = 0; g < kSplitGroups; g++) {
+      if (batch->split[g].jobs.empty()) continue;
+      launch_split_group(batch, g, precision, s);
+      staged = true;
     }
+    if (staged) launch_split_gather(batch, s);
     for (const fem_batch::Solo &j : batch->solo) {
       const int rc = fem::plan_assemble(j.plan, j.states, j.coords, j.E, j.nu, j.t, j.residual, j.values, precision, s,
                                         nullptr, false);

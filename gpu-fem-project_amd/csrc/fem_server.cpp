@@ -376,9 +376,7 @@ int fem_server_create(const fem_server_config *cfg, fem_server **server) {
     if (hipStreamCreateWithFlags(&slot.stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&slot.done, hipEventDisableTiming) != hipSuccess ||
         fem_batch_create(cfg->maxBatchJobs, cfg->useGraphs ? FEM_BATCH_GRAPH : 0, &slot.batch) != FEM_OK ||
-        fem::batch_prepare_graph(slot.batch, cfg->precision) != FEM_OK) {
-      // (graphs are recorded here, before the worker starts: a capture in flight would make other threads'
-      // default-stream work, such as fem_server_add_mesh's uploads, fail)
+        fem::batch_prepare(slot.batch, cfg->precision) != FEM_OK) {
       fem_server_destroy(s);
       return set_error(FEM_ERR_HIP, "creating server streams/events/batches failed");
     }
@@ -410,10 +408,10 @@ int fem_server_add_mesh(fem_server *server, int order, int numNodes, int numElem
                        &m.plan);
   if (rc) return rc;
   if (server->cfg.useGraphs && !fem::plan_streams_public(m.plan)) {
-    // A graph batch replays the streaming kernel, whose parts are one batch per wavefront; this mesh's parts
-    // are larger (a node shared by more elements than a workgroup takes at once).
+    // Such batches run the streaming kernel, whose parts are one batch per wavefront; this mesh's parts are
+    // larger (a node shared by more elements than a workgroup takes at once).
     fem_plan_destroy(m.plan);
-    return set_error(FEM_ERR_UNSUPPORTED, "the mesh's parts do not fit the graph-replayed batch kernel; "
+    return set_error(FEM_ERR_UNSUPPORTED, "the mesh's parts do not fit the batch kernel; "
                      "create the server with useGraphs = 0 to serve it");
   }
   int64_t planBytes = 0;

@@ -275,7 +275,7 @@ int fem_plan_destroy(fem_plan *plan);
  * Many assemblies on many resident plans in one call: jobs are grouped by element order and outputs
  * and each group runs as ONE persistent launch over all of its meshes' parts (no per-mesh launches).
  * Jacobian jobs of orders 3-4 run element-once (see fem_plan_create): one persistent launch per order
- * and residual/no-residual group, then the gathers, with staging in the batch's own device arena (grown
+ * and residual/no-residual group, then one launch of all gathers, with staging in the batch's own device arena (grown
  * at assembly when the batch's jobs need more, after a device synchronisation), so batches holding the
  * same plans may run concurrently on different streams.
  * Pointers are the same as fem_plan_assemble's; outputs are overwritten. Jobs of plans built with
@@ -285,8 +285,9 @@ int fem_plan_destroy(fem_plan *plan);
  * tables (asynchronously on `stream`) and launches; the batch may be cleared and refilled once the call
  * returns. */
 typedef struct fem_batch fem_batch;
-/* maxJobs: capacity per (order, outputs) group. flags: FEM_BATCH_GRAPH replays the twelve group
- * launches as one captured hipGraph whose kernels read their job counts from device memory. */
+/* maxJobs: capacity per (order, outputs) group. flags: FEM_BATCH_GRAPH takes only jobs that run in the groups' own
+ * launches, so that a call's launches do not grow with its jobs. (The launches of the groups that hold jobs are issued
+ * directly: a recorded graph of all groups' launches is slower at every composition, also with all groups in use.) */
 int fem_batch_create(int maxJobs, int flags, fem_batch **batch);
 #define FEM_BATCH_GRAPH 1
 int fem_batch_clear(fem_batch *batch);
@@ -311,13 +312,13 @@ typedef struct fem_server_config {
   int maxBatchJobs;       /* jobs per (order, outputs) group in one batch */
   int numSlots;           /* batches in flight (streams), 1..8 */
   int precision;          /* FEM_PREC_FP64 or FEM_PREC_MIXED */
-  int useGraphs;          /* replay each batch's launches through a captured hipGraph */
+  int useGraphs;          /* batches are FEM_BATCH_GRAPH; their kernels are loaded when the server is created */
 } fem_server_config;
 
 int fem_server_create(const fem_server_config *cfg, fem_server **server);
 /* Builds the mesh's BSR pattern and resident plan (host arrays in, as fem_plan_create) and uploads its
  * coordinates. FEM_ERR_BUDGET if it does not fit; FEM_ERR_UNSUPPORTED (with useGraphs) if its parts do not
- * fit the graph-replayed kernel. */
+ * fit the batch kernel. */
 int fem_server_add_mesh(fem_server *server, int order, int numNodes, int numElements, const int *connPtr,
                         const int *conn, const double *nodeCoordsHost, double E, double nu, double t, int *meshId);
 int fem_server_mesh_info(fem_server *server, int meshId, int64_t *numNodes, int64_t *numBlocks,

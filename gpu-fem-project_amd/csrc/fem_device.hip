@@ -1296,9 +1296,13 @@ struct MeshJob {
   const uint16_t *visitRow;  // residual-only plans: [visits*N] part-local row of each visit's nodes, or kNoRow
 };
 
+// One job travels in the kernel's arguments: a table in device memory costs a dependent load in every workgroup and,
+// whenever the caller's buffers change, a copy before the launch (4096 bilinear elements: 8.6 us a call with the table
+// and 8.2 without; with other buffers on every call 11.2 and 8.3).
 struct OwnerArgs {
-  const MeshJob *jobs;    // device job table
-  const int *jobStart;    // [numJobs+1] first global part of each job
+  MeshJob job;            // the job, if jobs is NULL
+  const MeshJob *jobs;    // streaming kernel: a device job table (a batch)
+  const int *jobStart;    // [numJobs+1] first global part of each job of the table
   int numJobs;
   int totalParts;
   Basis1D basis;
@@ -1846,16 +1850,16 @@ __device__ __forceinline__ void zero_planes(double *acc, int nb) {
 }
 
 // Residual-only plans: one workgroup per part, by lines of nodes, LDS sums per owned row, one store per row.
-// Bound by latency (701 x 699 order 2: VALU 40% and LDS 37% busy, 2.1 TB/s): 54 us against 148 for the kernel that
-// formed each node's gradient at every point (lane (el, node)) and looked the rows up per node; 67 us without the
-// loads running ahead and with parts of 1024 rows.
+// Bound by latency (701 x 699 order 2: VALU 40% and LDS 37% busy at 54 us): 44 us with the job in the arguments, 54
+// with one more dependent load for it, 67 without the loads running ahead and with parts of 1024 rows besides; 137 for
+// the kernel that formed each node's gradient at every point (lane (el, node)) and looked the rows up per node.
 template <int P, int MAXR>
 __global__ __launch_bounds__(kLineWaves * 64) void residual_part_kernel(const OwnerArgs args) {
   using O = LineOrd<P>;
   constexpr int NP = O::NP, N = O::N, THREADS = kLineWaves * 64;
   __shared__ __align__(16) double exAll[kLineWaves][O::EPW * O::EL];
   __shared__ __align__(16) double racc[2 * MAXR];
-  const MeshJob &J = args.jobs[0];
+  const MeshJob &J = args.job;
   const int per = int(gridDim.x) / 8;  // contiguous parts per XCD, as in owner_kernel
   const int part = int(blockIdx.x % 8) * per + int(blockIdx.x / 8);
   if (part >= args.totalParts) return;
@@ -1935,7 +1939,7 @@ __global__ __launch_bounds__(WAVES * 64) void owner_kernel(const OwnerArgs args)
   __shared__ int lbase[MAXR];
   __shared__ int4 lruns[JAC ? MAXR : 1];
 
-  const MeshJob &J = args.jobs[0];
+  const MeshJob &J = args.job;
   // XCD-aware order: consecutive workgroup ids land on different XCDs, so give each XCD a
   // contiguous range of (spatially adjacent) parts to keep shared element data in its L2.
   const int per = int(gridDim.x) / 8;
@@ -2102,8 +2106,9 @@ __device__ __forceinline__ void stream_parts(const MeshJob &J, int p0, int p1, W
 
 // Streaming kernel for parts that take one batch per wavefront (the default partition), over one or
 // many jobs (a batch of resident meshes of one order). A persistent workgroup walks a contiguous range
-// of global parts, job by job; job fields and material sit in scalar registers for the job's parts.
-template <int P, typename T, int WAVES, int MAXB, int MAXR, bool RES, bool JAC>
+// of global parts, job by job; job fields and material sit in scalar registers for the job's parts. TABLE: the jobs of
+// a batch's table, else the one in the arguments.
+template <int P, typename T, int WAVES, int MAXB, int MAXR, bool RES, bool JAC, bool TABLE>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void owner_stream_kernel(const OwnerArgs args) {
   using O = Ord<P>;
@@ -2132,6 +2137,10 @@ void owner_stream_kernel(const OwnerArgs args) {
   fill_gref<P>(gref, args.basis);
   WaveLDS<P, T> &W = wl[threadIdx.x / 64];
 
+  if (!TABLE) {
+    stream_parts<P, T, WAVES, MAXB, MAXR, RES, JAC>(args.job, pb, pe, W, basis, gref, acc, racc, lrows, lbase, lruns);
+    return;
+  }
   // job of the first part: binary search of the job start table
   int j = 0;
   {
@@ -2452,8 +2461,9 @@ void launch_owner(const OwnerLaunch &L, hipStream_t stream) {
       // streamGrid is two workgroups per CU; 8-wave workgroups fill a CU's LDS alone.
       const int persistent = cfg.waves >= 8 ? std::max(8, L.streamGrid / 16 * 8) : L.streamGrid;
       const int grid = std::min(persistent, std::max((L.args.totalParts + 7) / 8, 1) * 8);
-      owner_stream_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC><<<grid, cfg.waves * 64, 0, stream>>>(
-          L.args);
+      auto *kernel = L.args.jobs ? owner_stream_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC, true>
+                                 : owner_stream_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC, false>;
+      kernel<<<grid, cfg.waves * 64, 0, stream>>>(L.args);
       return;
     }
   }
@@ -2607,7 +2617,7 @@ int alloc_doubles(int64_t n, double **d, int64_t &bytes) {
 
 void free_plan_arrays(fem_plan *p) {
   void *ptrs[] = {p->dVisitConn, p->dVisitEid, p->dVisitRow, p->dNodeLrow, p->dRows,  p->dRowLbase, p->dRuns,  p->dColourOff,
-                  p->dPartDesc,  p->dRank,     p->dJob,      p->dJobStart, p->dConn,   p->dCode,  p->dRcode,
+                  p->dPartDesc,  p->dRank,     p->dConn,   p->dCode,  p->dRcode,
                   p->dGline,     p->dGptr,     p->dGsrc,     p->dRline,  p->dRptr,     p->dRsrc,  p->dStage,
                   p->dRstage};
   for (void *q : ptrs) {
@@ -2786,14 +2796,13 @@ int create_plan(int order, int numNodes, int numElements, const int *connPtr, co
   p->maxPartRows = h.maxPartRows;
   (void)hipGetDevice(&p->device);
   if (hipDeviceGetAttribute(&p->numCUs, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess) p->numCUs = 0;
-  const std::vector<int> jobStart = {0, h.numParts};
   int64_t bytes = 0;
   if ((rc = upload(h.visitConn, &p->dVisitConn, bytes)) || (rc = upload(h.visitEid, &p->dVisitEid, bytes)) ||
       (rc = upload(h.visitRow, &p->dVisitRow, bytes)) ||
       (rc = upload(h.nodeLrow, &p->dNodeLrow, bytes)) || (rc = upload(h.rows, &p->dRows, bytes)) ||
       (rc = upload(h.rowLbase, &p->dRowLbase, bytes)) || (rc = upload(h.runs, &p->dRuns, bytes)) ||
       (rc = upload(h.colourOff, &p->dColourOff, bytes)) || (rc = upload(h.partDesc, &p->dPartDesc, bytes)) ||
-      (rc = upload(h.rank, &p->dRank, bytes)) || (rc = upload(jobStart, &p->dJobStart, bytes))) {
+      (rc = upload(h.rank, &p->dRank, bytes))) {
     free_plan_arrays(p);
     delete p;
     return rc;
@@ -2830,13 +2839,6 @@ int create_plan(int order, int numNodes, int numElements, const int *connPtr, co
       clear_error();
     }
   }
-  if (hipMalloc(reinterpret_cast<void **>(&p->dJob), sizeof(MeshJob)) != hipSuccess) {
-    free_plan_arrays(p);
-    delete p;
-    return set_error(FEM_ERR_OUT_OF_MEMORY, "hipMalloc of the plan's job record failed");
-  }
-  bytes += int64_t(sizeof(MeshJob));
-  static_assert(sizeof(MeshJob) <= sizeof(p->hostJob), "job record size");
   p->deviceBytes = bytes;
   p->partScale = partScale;
   p->flags = flags & ~FEM_PLAN_AUTOTUNE;
@@ -3005,16 +3007,8 @@ int fem::plan_assemble(fem_plan *plan, const double *states, const double *nodeC
   OwnerLaunch L{};
   if ((rc = make_basis(plan->order, L.args.basis))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // The device job record is rewritten only when the request's pointers or material change.
-  MeshJob job = make_job(plan, states, nodeCoords, residual, matEntries, m);
-  job.accumulate = accumulate ? 1 : 0;
-  if (!plan->jobUploaded || std::memcmp(&job, plan->hostJob, sizeof(MeshJob)) != 0) {
-    FEM_HIP_CHECK(hipMemcpyAsync(plan->dJob, &job, sizeof(MeshJob), hipMemcpyHostToDevice, s));
-    std::memcpy(plan->hostJob, &job, sizeof(MeshJob));
-    plan->jobUploaded = true;
-  }
-  L.args.jobs = reinterpret_cast<const MeshJob *>(plan->dJob);
-  L.args.jobStart = plan->dJobStart;
+  L.args.job = make_job(plan, states, nodeCoords, residual, matEntries, m);
+  L.args.job.accumulate = accumulate ? 1 : 0;
   L.args.numJobs = 1;
   L.args.totalParts = plan->numParts;
   L.precision = precision;
@@ -3442,7 +3436,8 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
         // Parts too large for streaming: one per-part launch per job.
         for (size_t j = 0; j < g.jobs.size(); j++) {
           OwnerLaunch Lj = L;
-          Lj.args.jobs = L.args.jobs + j;
+          Lj.args.job = g.jobs[j];
+          Lj.args.jobs = nullptr;
           Lj.args.numJobs = 1;
           Lj.args.totalParts = g.jobs[j].numParts;
           launch_owner_any(gi / 3 + 1, Lj, s);

@@ -159,7 +159,6 @@ struct fem_plan {
   int *dColourOff = nullptr;
   int *dPartDesc = nullptr;
   uint8_t *dRank = nullptr;
-  int *dJobStart = nullptr;  // {0, numParts}
   // Element-once assembly of Jacobian plans of orders 3-4 (SplitHost): connectivity, codes, gather lists and
   // staging arrays. dConn is NULL when the plan has none.
   int *dConn = nullptr;      // [E][N]
@@ -174,9 +173,6 @@ struct fem_plan {
   double partScale = 1.0;    // part budgets relative to the kernel's (FEM_PLAN_AUTOTUNE picks it)
   double tunedSeconds = 0;   // measured assembly time of the chosen build (autotuned plans)
   int tiledWaves = 4;        // orders 3-4: wavefronts per workgroup of the element-once kernel (autotuned)
-  void *dJob = nullptr;      // device job record of the last assembly
-  alignas(8) unsigned char hostJob[256] = {};  // host copy of that record
-  bool jobUploaded = false;
   int maxPartVisits = 0, maxPartRows = 0;
   int numCUs = 0;
 };

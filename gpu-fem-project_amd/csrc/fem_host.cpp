@@ -42,10 +42,10 @@ int hardware_threads() {
   return int(std::min(n, 64u));
 }
 
-// Runs fn(begin, end) over [0, n) split across threads.
+// Runs fn(begin, end) over [0, n) split across threads, each with at least `grain` of them.
 template <typename Fn>
-void parallel_for(int64_t n, Fn fn) {
-  const int nt = int(std::min<int64_t>(hardware_threads(), std::max<int64_t>(1, n / 4096)));
+void parallel_for(int64_t n, Fn fn, int64_t grain = 4096) {
+  const int nt = int(std::min<int64_t>(hardware_threads(), std::max<int64_t>(1, n / grain)));
   if (nt <= 1) {
     fn(int64_t(0), n);
     return;
@@ -540,7 +540,7 @@ void plan_gather(int64_t outputs, int unitsPerLine, std::vector<int> &code, cons
       for (int64_t i = c * kChunk; i < std::min(n, (c + 1) * kChunk); i++) count += staged(code[size_t(i)]);
       start[size_t(c) + 1] = count;
     }
-  });
+  }, 1);
   for (int64_t c = 0; c < chunks; c++) start[size_t(c) + 1] += start[size_t(c)];
   out.slots = start[size_t(chunks)];
   parallel_for(chunks, [&](int64_t b, int64_t e) {
@@ -556,7 +556,7 @@ void plan_gather(int64_t outputs, int unitsPerLine, std::vector<int> &code, cons
         }
       }
     }
-  });
+  }, 1);
   out.line.clear();
   out.ptr.assign(1, 0);
   out.src.clear();

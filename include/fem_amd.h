@@ -101,8 +101,9 @@ int fem_bsr_pattern_cols(int numNodes, int numElements, int nodesPerElement, con
  * (FEM_ERR_MAP_MISS), not a printed warning with the entry left unset (TACSHelpers.h:176-178). */
 int fem_element_bcsr_map(const int *connPtr, const int *conn, int numElements, int nodesPerElement, int numRows,
                          const int *rowp, const int *cols, int bsize, int *map);
-/* Element-once tables of a mesh on the host: what fem_plan_create builds for Jacobian assemblies of orders
- * 3-4 (any order here). code[(e*N + a)*N + b] is the BSR index of block (conn[e,a], conn[e,b]) when element e
+/* Element-once tables of a mesh on the host: what fem_plan_create's tables for Jacobian assemblies of orders 3-4 are
+ * made from (any order here; a plan then stores each output's first contribution in place and groups the other slots
+ * by 64-byte lines of the output). code[(e*N + a)*N + b] is the BSR index of block (conn[e,a], conn[e,b]) when element e
  * alone forms it, else numBlocks + a staging slot; rcode[e*N + a] likewise for node conn[e,a]'s residual,
  * against numNodes. gdst / gptr list the other blocks (ascending) and their slot ranges (gptr has
  * *numGather + 1 entries), rdst / rptr the other nodes. Each output is the sum of its slots in slot order

@@ -2124,7 +2124,7 @@ void owner_stream_kernel(const OwnerArgs args) {
   __shared__ int2 lruns[JAC ? 2 : 1][MAXR];
 
   // Contiguous range of global parts per workgroup; workgroup w runs on XCD w % 8, and each XCD's
-  // workgroups share one contiguous (spatially adjacent, Morton-ordered) stretch of parts.
+  // workgroups share one contiguous (spatially adjacent) stretch of parts.
   const int xcd = int(blockIdx.x % 8), slot = int(blockIdx.x / 8), perX = int(gridDim.x / 8);
   const int numJobs = args.numJobs;
   const int64_t np = args.totalParts;

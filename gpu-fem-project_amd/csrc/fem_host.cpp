@@ -251,7 +251,9 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
   // the elements' centres, else natural. A part costs one round of the workgroup whatever it holds, and an element is
   // visited by every part that owns one of its nodes, so compact parts are what counts: 1.44-1.53 visits an element at
   // order 2 and 1.27-1.31 at order 1, where a Morton curve through the nodes gave 1.50-1.62 and 1.32-1.36 (its jumps
-  // cut parts in two) and a Hilbert curve through the nodes 1.45-1.56 and 1.29-1.33 (it cuts through elements).
+  // cut parts in two) and a Hilbert curve through the nodes 1.45-1.56 and 1.29-1.33 (it cuts through elements). Owner
+  // Jacobians of orders 3-4 form only the rows a part owns, so there a curve through the nodes is the better one (order 4,
+  // annulus 60 x 300, mixed: 351 us against 383; the Morton curve's 359).
   std::vector<int> order_nodes(numNodes);
   std::iota(order_nodes.begin(), order_nodes.end(), 0);
   if (nodeCoords) {
@@ -264,8 +266,12 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
     }
     const double sx = xmax > xmin ? 65535.0 / (xmax - xmin) : 0.0;
     const double sy = ymax > ymin ? 65535.0 / (ymax - ymin) : 0.0;
-    std::vector<uint32_t> code(numElements);
-    parallel_for(numElements, [&](int64_t b, int64_t e) {
+    auto cell = [&](double x, double y) {
+      return hilbert2(uint32_t(std::lround((x - xmin) * sx)), uint32_t(std::lround((y - ymin) * sy)));
+    };
+    const bool byNode = order >= 3 && (flags & FEM_PLAN_OWNER_ONLY) != 0;
+    std::vector<uint32_t> code(byNode ? 0 : numElements);
+    parallel_for(int64_t(code.size()), [&](int64_t b, int64_t e) {
       for (int64_t el = b; el < e; el++) {
         const int *en = conn + connPtr[el];
         double x = 0, y = 0;
@@ -273,14 +279,15 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
           x += nodeCoords[2 * int64_t(en[i])];
           y += nodeCoords[2 * int64_t(en[i]) + 1];
         }
-        code[size_t(el)] = hilbert2(uint32_t(std::lround((x / N - xmin) * sx)), uint32_t(std::lround((y / N - ymin) * sy)));
+        code[size_t(el)] = cell(x / N, y / N);
       }
     });
     std::vector<uint64_t> key(numNodes);
     parallel_for(numNodes, [&](int64_t b, int64_t e) {
       for (int64_t n = b; n < e; n++) {
         uint32_t first = UINT32_MAX;
-        for (int j = nptr[n]; j < nptr[n + 1]; j++) first = std::min(first, code[size_t(nadj[size_t(j)])]);
+        if (byNode) first = cell(nodeCoords[2 * n], nodeCoords[2 * n + 1]);
+        else for (int j = nptr[n]; j < nptr[n + 1]; j++) first = std::min(first, code[size_t(nadj[size_t(j)])]);
         key[size_t(n)] = (uint64_t(first) << 32) | uint32_t(n);
       }
     });

@@ -154,7 +154,7 @@ def rel_err(torch, a, b):
 
 
 def bench_batch(args, F, torch):
-    """256 meshes assembled by one batch call (one persistent launch per order/output group, graph replay)
+    """256 meshes assembled by one batch call (one persistent launch per order/output group)
     against one plan launch per mesh and against plain FP64 per-mesh atomic launches."""
     dev = torch.device("cuda:0")
     count = args.pool or 256
@@ -306,8 +306,8 @@ def wait_until(t):
 
 
 def bench_serve(args, F, torch):
-    """Poisson arrivals over 64 resident meshes: the serving loop (mixed precision, continuous batching, graph
-    replay) against plain FP64 per-request launches (FIFO, one request at a time, residual and Jacobian as
+    """Poisson arrivals over 64 resident meshes: the serving loop (mixed precision, continuous batching)
+    against plain FP64 per-request launches (FIFO, one request at a time, residual and Jacobian as
     separate element-parallel atomic launches). Latency = completion - scheduled arrival."""
     import threading
     import queue
@@ -403,7 +403,7 @@ def bench_serve(args, F, torch):
     mesh_ids, jacs, unit_arrivals = request_stream(F, max(n_main, args.side_requests), 7, pool_size)
     elems = np.array([m.num_elements for m in meshes])
 
-    # Warm-up: every mesh once each way on both paths (graph capture, output-pool fill).
+    # Warm-up: every mesh once each way on both paths (output-pool fill).
     for k in range(pool_size):
         for jac in (False, True):
             plain_one(k, jac, 0)
@@ -691,7 +691,7 @@ def serve_leg(args, F, torch):
 
 
 def batch_leg(args, F, torch):
-    """C4 leg of the default run: bench_batch (256 meshes, mixed precision, autotuned plans, graph replay)."""
+    """C4 leg of the default run: bench_batch (256 meshes, mixed precision, autotuned plans)."""
     import contextlib
     import io
 

@@ -268,8 +268,9 @@ int fem_jacobian_dropin(int order, const int *connPtr, const int *conn, int numE
   };
   if (order < 1 || order > 2 || numElements <= 0 || !connPtr || !conn || !elementBCSRMap || !matEntries || !states ||
       !nodeCoords || (precision != FEM_PREC_FP64 && precision != FEM_PREC_MIXED)) {
-    // argument errors are reported by fem_jacobian; at orders 3-4 its atomic kernels are faster than the
-    // element-once route in accumulate mode (annulus 200x1250 order 4: 4.3 against 6.0 ms)
+    // argument errors are reported by fem_jacobian. Orders 3-4 stay without a cached plan: in accumulate mode it is
+    // faster (annulus 200x1250 order 4: 3.1 against 4.3 ms of atomics), but a first call would take the seconds and
+    // the 1.4 GB of its tables and staging
     return plain();
   }
   if (int64_t(numElements) * nodes_per_element(order) * nodes_per_element(order) > INT32_MAX) return plain();

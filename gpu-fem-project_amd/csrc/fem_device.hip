@@ -1149,12 +1149,18 @@ __device__ __forceinline__ void stage_geometry_nl(WaveLDSNL<P> &W, const Basis1D
 // gradients of the chunk's rows come through the per-wave LDS one quadrature point at a time. All lanes of
 // the wavefront must call this; `valid` masks the lane's writes. Every lane calls emit(at, k) for every row,
 // in step, with a negative destination when it has none (so emit may exchange values across lanes).
+// Every chunk forms the lane's own terms of every point again and pads its last rows, and the LDS allows two wavefronts
+// per SIMD whatever the registers, so CH is the size that leaves few chunks and little padding: 2 of 5 for 9 rows, 2 of
+// 8 for 16, 5 of 5 for 25. Against 4 rows at every order: 324 -> 321 us (90 300 quadratic elements), 550 -> 547
+// (58 563 cubic), 1143 -> 1028 (40 200 quartic, 4 chunks of 7: 1057; 2 of 13 spill: 7.8 ms). Orders 1-3 are near the
+// bound of their atomic requests, order 4 is not (788 us).
 template <int P, typename Where, typename Emit>
 __device__ __forceinline__ void stage_stiffness_nl(WaveLDSNL<P> &W, const double2 *gref, const Material &m, int el,
                                                    int b, bool valid, double &Rx, double &Ry, Where &&where,
                                                    Emit &&emit) {
   using O = Ord<P>;
-  constexpr int N = O::N, Q = O::Q, NG = WaveLDSNL<P>::NG, CH = 4;
+  constexpr int N = O::N, Q = O::Q, NG = WaveLDSNL<P>::NG;
+  constexpr int CH = P == 3 ? 8 : P == 1 ? 4 : 5;
   const int elc = el < O::EPW ? el : O::EPW - 1;
   const int bc = b < N ? b : 0;
   const double mu = m.mu, lam = m.lambda;

@@ -1453,7 +1453,7 @@ __device__ __forceinline__ void rows_chunk(WaveLDS<P, T> &W, const double2 *gref
 }
 
 // Row-restricted stiffness (orders >= 3, where an element is visited by several parts): lane (el, b) forms
-// K(a, b) only for the rows a this part owns, W.orow[el][0..count), in chunks of 8 rows (4 in FP64; maxCount,
+// K(a, b) only for the rows a this part owns, W.orow[el][0..count), in chunks of 8 rows (4 or 5 in FP64; maxCount,
 // the largest count over the wavefront's elements, sets the number of chunks). Over all parts visiting an
 // element this forms each row of K_e once, instead of the whole symmetric K_e per visit. The residual of
 // node b is accumulated in the first chunk. where and emit as for stage_stiffness, except that emit gets a
@@ -1463,7 +1463,10 @@ template <int P, typename T, bool JAC, bool ALL_LANES, typename Where, typename 
 __device__ __forceinline__ void stage_stiffness_rows(WaveLDS<P, T> &W, const double2 *gref, const Material &m, int el,
                                                      int b, bool valid, int count, int maxCount, double &Rx,
                                                      double &Ry, Where &&where, Emit &&emit) {
-  constexpr int CH = sizeof(T) == 8 ? 4 : 8;  // FP64 chunks are halved to stay within 256 registers
+  // FP64 chunks are halved to stay within 256 registers; 5 rows divide order 4's 25 (30 625 elements through atomics: 693
+  // us with 4 rows, 684 with 5, 688 with 8; owner-only plan of the annulus 60 x 300: 466 against 439), at order 3 4 rows
+  // are better than 8 (516 against 521 us).
+  constexpr int CH = sizeof(T) == 8 ? (P == 4 ? 5 : 4) : 8;
   Rx = 0;
   Ry = 0;
   const int chunks = JAC ? uniform(max((maxCount + CH - 1) / CH, 1)) : 1;

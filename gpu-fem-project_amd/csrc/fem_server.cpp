@@ -4,8 +4,7 @@
 // assembly requests (mesh, device states, residual-only or residual+Jacobian); the server allocates
 // each request's outputs when the request is admitted under the device-memory budget and keeps them
 // until the client releases them. A worker thread forms batches from the admitted requests and launches
-// each batch as fem_batch_assemble (one persistent launch per element order and output set, optionally
-// replayed through a captured hipGraph) on one of several streams ("slots"): requests that arrive while
+// each batch as fem_batch_assemble (one persistent launch per element order and output set) on one of several streams ("slots"): requests that arrive while
 // earlier batches run are collected into the next batch, which starts on a free slot and overlaps the
 // running ones on the device.
 //

@@ -300,13 +300,14 @@ __device__ __forceinline__ int find_col(const int *cols, int b, int e, int col) 
   return b;
 }
 
-// The map, one thread per entry (elements of another number of nodes than element_map_staged takes).
+// The map, one thread per entry (elements of another number of nodes than element_map_staged takes). maxBlocks: the
+// blocks whose bs2 entries each 32-bit offsets reach (0 where one block is too many); a larger pattern gets no map.
 __global__ __launch_bounds__(kThreads) void element_map(int numRows, int numElements, int npe, const int *connPtr,
                                                         const int *conn, const int *rowp, const int *cols, int bs2,
-                                                        int *map, int *flags) {
+                                                        int maxBlocks, int *map, int *flags) {
   const int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t nn = int64_t(npe) * npe;
-  if (int64_t(rowp[numRows]) * bs2 > INT32_MAX) {
+  if (rowp[numRows] > maxBlocks) {
     flags[kOverflow] = 1;
     return;
   }
@@ -339,10 +340,10 @@ struct MapTile {
 template <int NPE>
 __global__ __launch_bounds__(kThreads) void element_map_staged(int numRows, int numElements, const int *connPtr,
                                                                const int *conn, const int *rowp, const int *cols,
-                                                               int bs2, int *map, int *flags) {
+                                                               int bs2, int maxBlocks, int *map, int *flags) {
   constexpr int CAP = MapTile<NPE>::CAP, PER = MapTile<NPE>::PER, ROWS = MapTile<NPE>::ROWS;
   __shared__ int node[ROWS], begin[ROWS], count[ROWS], col[ROWS * CAP];
-  if (int64_t(rowp[numRows]) * bs2 > INT32_MAX) {
+  if (rowp[numRows] > maxBlocks) {
     flags[kOverflow] = 1;
     return;
   }
@@ -704,11 +705,13 @@ extern "C" int fem_element_bcsr_map_device(const int *connPtr, const int *conn, 
   int rc = sc.alloc(kFlags * sizeof(int));
   if (rc) return rc;
   int *flags = static_cast<int *>(sc.b.p);
+  const int64_t entries = int64_t(bsize) * bsize;  // of a block: beyond 32 bits from bsize 46341 on
+  const int maxBlocks = int(INT32_MAX / entries), bs2 = int(std::min<int64_t>(entries, INT32_MAX));
   fill_zero<<<1, kThreads, 0, stream>>>(flags, kFlags);
   auto staged = [&](auto npe) {
     constexpr int NPE = decltype(npe)::value, PER = MapTile<NPE>::PER;
     element_map_staged<NPE><<<unsigned((int64_t(numElements) + PER - 1) / PER), kThreads, 0, stream>>>(
-        numRows, numElements, connPtr, conn, rowp, cols, bsize * bsize, map, flags);
+        numRows, numElements, connPtr, conn, rowp, cols, bs2, maxBlocks, map, flags);
   };
   switch (nodesPerElement) {
     case 4: staged(std::integral_constant<int, 4>{}); break;
@@ -718,7 +721,7 @@ extern "C" int fem_element_bcsr_map_device(const int *connPtr, const int *conn, 
     default: {
       const int64_t n = int64_t(numElements) * nodesPerElement * nodesPerElement;
       element_map<<<grid_for(n), kThreads, 0, stream>>>(numRows, numElements, nodesPerElement, connPtr, conn, rowp,
-                                                        cols, bsize * bsize, map, flags);
+                                                        cols, bs2, maxBlocks, map, flags);
     }
   }
   FEM_HIP_CHECK(hipGetLastError());
@@ -727,8 +730,8 @@ extern "C" int fem_element_bcsr_map_device(const int *connPtr, const int *conn, 
   FEM_HIP_CHECK(hipStreamSynchronize(stream));
   sc.done = true;
   if (h[kOverflow]) {  // nothing was written
-    return set_error(FEM_ERR_UNSUPPORTED, "the pattern's blocks x %d entries overflow the map's 32-bit offsets",
-                     bsize * bsize);
+    return set_error(FEM_ERR_UNSUPPORTED, "the pattern's blocks x %lld entries overflow the map's 32-bit offsets",
+                     (long long)entries);
   }
   return report_flags(h);
 }

@@ -300,18 +300,20 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
   const double scale = std::min(1.0, std::max(partScale, 0.01));
   const int maxVisits = residualOnly ? (1 << 30) : std::max(1, int(cfg.maxVisits * scale));
   const int blockBudget = residualOnly ? maxBlocks : std::max(out.maxRowLength, int(maxBlocks * scale));
-  // Residual-only plans of the line kernel are cut smaller (rowBudget) than their parts may become when nodes of no
-  // element join them (joinBudget); where those do not fit, everything is cut at the largest size.
+  // A part may be cut smaller (cutRows, cutBlocks) than it may become when nodes of no element join it (rowBudget,
+  // blockBudget), as residual-only plans of the line kernel are.
   const bool linePlan = residualOnly && !(flags & FEM_PLAN_DETERMINISTIC);
   int rowBudget = residualOnly ? maxRows : std::max(1, int(maxRows * scale));
-  int joinBudget = rowBudget;
+  int cutRows = rowBudget, cutBlocks = blockBudget;
   if (linePlan) {
-    joinBudget = residual_rows(order);
-    rowBudget = std::min(joinBudget, std::max(128, numNodes / 256));
+    rowBudget = residual_rows(order);
+    cutRows = std::min(rowBudget, std::max(128, numNodes / 256));
   }
   // Nodes that belong to no element keep zero blocks and zero residual entries. The cut runs over the other
   // nodes, so every part visits at least one element; each of them then joins the first part (in cut order)
-  // with room for its row, whose write-out stores the zeros.
+  // with room for its row, whose write-out stores the zeros. Where they do not all fit, the cut is made again with
+  // more room beside it: parts of the line kernel's largest size, then cuts of half the rows and blocks, down to
+  // one row (97 x 101 elements of order 2 hold 32 831 such nodes as first cut).
   std::vector<int> isolated;
   {
     std::vector<int> kept;
@@ -334,7 +336,7 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
       int newVisits = 0;
       for (int j = nptr[n]; j < nptr[n + 1]; j++) newVisits += stamp[nadj[size_t(j)]] != part;
       if (rowsInPart > 0 &&
-          (blocks + len > blockBudget || rowsInPart + 1 > rowBudget || visits + newVisits > maxVisits)) {
+          (blocks + len > cutBlocks || rowsInPart + 1 > cutRows || visits + newVisits > maxVisits)) {
         cutPtr.push_back(k);
         partRowCount.push_back(rowsInPart);
         partBlockCount.push_back(blocks);
@@ -357,7 +359,7 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
     int p = 0, unplaced = -1;
     for (int n : isolated) {
       const int len = rowp[n + 1] - rowp[n];
-      while (p < cutParts && (partRowCount[p] + 1 > joinBudget || partBlockCount[p] + len > blockBudget)) p++;
+      while (p < cutParts && (partRowCount[p] + 1 > rowBudget || partBlockCount[p] + len > blockBudget)) p++;
       if (p == cutParts) {
         unplaced = n;
         break;
@@ -367,11 +369,15 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
       partBlockCount[p] += len;
     }
     if (unplaced < 0) break;
-    if (!linePlan || rowBudget == maxRows) {
+    if (linePlan && rowBudget < maxRows) {
+      cutRows = rowBudget = maxRows;
+    } else if (cutRows > 1) {
+      cutRows /= 2;
+      cutBlocks = std::max(cutBlocks / 2, 1);
+    } else {
       return set_error(FEM_ERR_UNSUPPORTED, "no part has room for the row of node %d, which belongs to no element",
                        unplaced);
     }
-    rowBudget = joinBudget = maxRows;
   }
   {
     const int cutParts = int(cutPtr.size()) - 1;

@@ -2611,7 +2611,7 @@ int check_common(int order, const int *connPtr, const int *conn, int numElements
 template <typename TPtr>
 int upload(const std::vector<TPtr> &h, TPtr **d, int64_t &bytes) {
   const size_t n = std::max<size_t>(h.size(), 1) * sizeof(TPtr);
-  FEM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(d), n));
+  FEM_HIP_CHECK(hipError_t(device_alloc(reinterpret_cast<void **>(d), n)));
   if (!h.empty()) FEM_HIP_CHECK(hipMemcpy(*d, h.data(), h.size() * sizeof(TPtr), hipMemcpyHostToDevice));
   bytes += int64_t(n);
   return FEM_OK;
@@ -2619,7 +2619,7 @@ int upload(const std::vector<TPtr> &h, TPtr **d, int64_t &bytes) {
 
 int alloc_doubles(int64_t n, double **d, int64_t &bytes) {
   const size_t sz = size_t(std::max<int64_t>(n, 1)) * sizeof(double);
-  FEM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(d), sz));
+  FEM_HIP_CHECK(hipError_t(device_alloc(reinterpret_cast<void **>(d), sz)));
   bytes += int64_t(sz);
   return FEM_OK;
 }
@@ -2887,10 +2887,10 @@ int fem_plan_create(int order, int numNodes, int numElements, const int *connPtr
   TuneBuffers tb;
   const size_t nb = size_t(rowp[numNodes]);
   FEM_HIP_CHECK(hipStreamCreateWithFlags(&tb.stream, hipStreamNonBlocking));
-  FEM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&tb.coords), size_t(numNodes) * 16));
-  FEM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&tb.states), size_t(numNodes) * 16));
-  FEM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&tb.res), size_t(numNodes) * 16));
-  FEM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&tb.vals), nb * 32));
+  FEM_HIP_CHECK(hipError_t(device_alloc(reinterpret_cast<void **>(&tb.coords), size_t(numNodes) * 16)));
+  FEM_HIP_CHECK(hipError_t(device_alloc(reinterpret_cast<void **>(&tb.states), size_t(numNodes) * 16)));
+  FEM_HIP_CHECK(hipError_t(device_alloc(reinterpret_cast<void **>(&tb.res), size_t(numNodes) * 16)));
+  FEM_HIP_CHECK(hipError_t(device_alloc(reinterpret_cast<void **>(&tb.vals), nb * 32)));
   FEM_HIP_CHECK(hipMemcpy(tb.coords, nodeCoordsHost, size_t(numNodes) * 16, hipMemcpyHostToDevice));
   FEM_HIP_CHECK(hipMemset(tb.states, 0, size_t(numNodes) * 16));
   fem_plan *best = nullptr;
@@ -3231,7 +3231,7 @@ int fem_batch_create(int maxJobs, int flags, fem_batch **batch) {
   b->splitStartOffset = b->jobsOffset + G * size_t(maxJobs) * sizeof(MeshJob);
   b->splitJobsOffset = (b->splitStartOffset + SG * 3 * size_t(maxJobs + 1) * sizeof(int) + 255) / 256 * 256;
   b->tableBytes = b->splitJobsOffset + SG * size_t(maxJobs) * sizeof(SplitJob);
-  if (hipMalloc(reinterpret_cast<void **>(&b->dTables), b->tableBytes) != hipSuccess ||
+  if (device_alloc(reinterpret_cast<void **>(&b->dTables), b->tableBytes) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void **>(&b->hTables), b->tableBytes, hipHostMallocDefault) != hipSuccess ||
       hipEventCreateWithFlags(&b->staged, hipEventDisableTiming) != hipSuccess) {
     free_batch(b);
@@ -3383,11 +3383,10 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
     batch->dArena = nullptr;
     batch->arenaDoubles = 0;
     for (const int64_t n : {want, batch->splitDoubles}) {
-      if (hipMalloc(reinterpret_cast<void **>(&batch->dArena), size_t(n) * sizeof(double)) == hipSuccess) {
+      if (device_alloc(reinterpret_cast<void **>(&batch->dArena), size_t(n) * sizeof(double)) == hipSuccess) {
         batch->arenaDoubles = n;
         break;
       }
-      (void)hipGetLastError();
       batch->dArena = nullptr;
     }
     if (!batch->dArena) {

@@ -155,7 +155,7 @@ struct Temp {
   template <typename T>
   int alloc(T **out, size_t n) {
     void *q = nullptr;
-    if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) {
+    if (device_alloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) {
       return set_error(FEM_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes failed", n * sizeof(T));
     }
     p.push_back(q);

@@ -118,6 +118,9 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
 
 // Frees the idle scratch that the device pattern and map builders keep (fem_pattern.hip); returns the blocks freed.
 int pattern_scratch_clear();
+// hipMalloc for all of the library's device memory: where there is no room it first frees that scratch. Returns the
+// hipError_t and leaves no error pending.
+int device_alloc(void **p, size_t bytes);
 
 // Batches (fem_device.hip). Doubles of element-once staging a Jacobian job of `plan` takes (0: the plan has no
 // element-once tables); fem_batch_add with that staging owned by the caller (`stage`, NULL: the batch's own

@@ -418,11 +418,7 @@ struct Scratch {
         }
       }
     }
-    hipError_t e = hipMalloc(&b.p, bytes);
-    if (e != hipSuccess && pattern_scratch_clear() > 0) {
-      (void)hipGetLastError();
-      e = hipMalloc(&b.p, bytes);
-    }
+    const hipError_t e = hipError_t(device_alloc(&b.p, bytes));
     if (e != hipSuccess) {
       b.p = nullptr;
       return set_error(FEM_ERR_HIP, "hipMalloc of %zu bytes of pattern scratch failed: %s", bytes, hipGetErrorString(e));
@@ -742,4 +738,14 @@ int fem::pattern_scratch_clear() {
   for (const KeptBlock &b : kept) (void)hipFree(b.p);
   kept.clear();
   return n;
+}
+
+int fem::device_alloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && pattern_scratch_clear() > 0) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) (void)hipGetLastError();
+  return int(e);
 }

@@ -126,7 +126,7 @@ int64_t arena_need(const ServerMesh &m, bool withJacobian) {
 bool create_arena(fem_server *s, int64_t bytes) {
   bytes = bytes / kArenaAlign * kArenaAlign;
   if (bytes <= 0) return false;
-  if (hipMalloc(reinterpret_cast<void **>(&s->arena), size_t(bytes)) != hipSuccess) {
+  if (fem::device_alloc(reinterpret_cast<void **>(&s->arena), size_t(bytes)) != hipSuccess) {
     s->arena = nullptr;
     return false;
   }
@@ -427,7 +427,7 @@ int fem_server_add_mesh(fem_server *server, int order, int numNodes, int numElem
     }
     server->residentBytes += m.residentBytes;
   }
-  if (hipMalloc(reinterpret_cast<void **>(&m.coords), size_t(numNodes) * 16) != hipSuccess ||
+  if (fem::device_alloc(reinterpret_cast<void **>(&m.coords), size_t(numNodes) * 16) != hipSuccess ||
       hipMemcpy(m.coords, nodeCoordsHost, size_t(numNodes) * 16, hipMemcpyHostToDevice) != hipSuccess) {
     fem_plan_destroy(m.plan);
     std::lock_guard<std::mutex> lk(server->mu);

@@ -147,7 +147,8 @@ int fem_write_bdf(const char *path, int order, int numNodes, int numElements, co
  * replace the host set-up the reference leaves to TACS (createSchurMat, verification/TestKernels.cpp:105)
  * and generateElementBCSRMap (verification/TACSHelpers.h:138-182). Each call returns after its work has
  * finished. Scratch comes from one block per GPU that the library keeps (up to 256 MiB, released by
- * fem_dropin_cache_clear); calls that overlap, and larger meshes, allocate and free their own. connPtr entries must index valid conn entries, as for
+ * fem_dropin_cache_clear and when an allocation of the library finds no room); calls that overlap, and larger
+ * meshes, allocate and free their own. connPtr entries must index valid conn entries, as for
  * every entry point here.
  * fem_bsr_pattern_device fills rowp (numNodes + 1 entries) and *numBlocks. Pass cols = NULL to size the
  * pattern, then call again with cols of colsCapacity >= *numBlocks entries. FEM_ERR_UNSUPPORTED if a node's

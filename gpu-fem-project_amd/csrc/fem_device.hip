@@ -2806,6 +2806,10 @@ int create_plan(int order, int numNodes, int numElements, const int *connPtr, co
   (void)hipGetDevice(&p->device);
   if (hipDeviceGetAttribute(&p->numCUs, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess) p->numCUs = 0;
   int64_t bytes = 0;
+  if (!h.visitRow.empty()) {  // the line kernel of residual-only plans reads visitConn, visitRow, rows and partDesc
+    h.visitEid = h.nodeLrow = h.rowLbase = h.runs = h.colourOff = {};
+    h.rank = {};
+  }
   if ((rc = upload(h.visitConn, &p->dVisitConn, bytes)) || (rc = upload(h.visitEid, &p->dVisitEid, bytes)) ||
       (rc = upload(h.visitRow, &p->dVisitRow, bytes)) ||
       (rc = upload(h.nodeLrow, &p->dNodeLrow, bytes)) || (rc = upload(h.rows, &p->dRows, bytes)) ||

@@ -485,7 +485,7 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
       std::memcpy(&out.visitConn[size_t(v) * N], conn + connPtr[out.visitEid[size_t(v)]], N * sizeof(int));
     }
   });
-  if (residualOnly) {  // the part-local row of each visit's nodes, for the line kernel
+  if (linePlan) {  // the part-local row of each visit's nodes
     out.visitRow.resize(visits * N);
     parallel_for(P, [&](int64_t b, int64_t e) {
       for (int64_t p = b; p < e; p++) {

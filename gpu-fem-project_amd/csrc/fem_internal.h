@@ -59,7 +59,7 @@ struct PlanHost {
   int64_t numBlocks = 0;
   std::vector<int> visitConn;     // [visits*N] nodes of each element visit (parts' visits contiguous)
   std::vector<int> visitEid;      // [visits] element id of each visit
-  std::vector<uint16_t> visitRow; // [visits*N] residual-only plans: the node's row within the part, or kNoRow
+  std::vector<uint16_t> visitRow; // [visits*N] residual-only plans of the line kernel: the node's part row, or kNoRow
   std::vector<int> nodeLrow;      // [numNodes] index of the node within its part's row list
   std::vector<int> partRowPtr;    // [P+1]
   std::vector<int> rows;          // global row (node) ids, ascending within a part

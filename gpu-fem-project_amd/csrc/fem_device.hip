@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdio>
 #include <type_traits>
 #include <utility>
@@ -854,9 +855,9 @@ __device__ __forceinline__ int find_job(const int *start, int n, int64_t x) {
   return lo;
 }
 
-// A batch's element-once jobs of one order: counts = (jobs, units, staged blocks, staged residual entries)
-// in device memory, unitStart[j] the first unit of job j, a unit
-// being WAVES * EPW elements. Persistent: workgroups stride over the units.
+// A batch's element-once jobs of one order: counts = (jobs, units, block lines, residual lines) in device memory,
+// unitStart[j] the first unit of job j, a unit being WAVES * EPW elements. Persistent: workgroups stride over the
+// units.
 template <int P, typename T, int WAVES, bool RES>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(3)))
 void element_tiled_batch(const SplitJob *__restrict__ jobs, const int *__restrict__ unitStart,
@@ -1309,6 +1310,7 @@ struct OwnerArgs {
   MeshJob job;            // the job, if jobs is NULL
   const MeshJob *jobs;    // streaming kernel: a device job table (a batch)
   const int *jobStart;    // [numJobs+1] first global part of each job of the table
+  const int *counts;      // if not NULL: device (numJobs, totalParts), read instead of the two below
   int numJobs;
   int totalParts;
   Basis1D basis;
@@ -2135,8 +2137,8 @@ void owner_stream_kernel(const OwnerArgs args) {
   // Contiguous range of global parts per workgroup; workgroup w runs on XCD w % 8, and each XCD's
   // workgroups share one contiguous (spatially adjacent) stretch of parts.
   const int xcd = int(blockIdx.x % 8), slot = int(blockIdx.x / 8), perX = int(gridDim.x / 8);
-  const int numJobs = args.numJobs;
-  const int64_t np = args.totalParts;
+  const int numJobs = TABLE && args.counts ? cmem(args.counts)[0] : args.numJobs;
+  const int64_t np = TABLE && args.counts ? cmem(args.counts)[1] : args.totalParts;
   const int xb = int(np * xcd / 8), xe = int(np * (xcd + 1) / 8);
   const int pb = xb + int(int64_t(xe - xb) * slot / perX);
   const int pe = xb + int(int64_t(xe - xb) * (slot + 1) / perX);
@@ -2378,6 +2380,7 @@ constexpr int kSplitGroups = 4;
 struct BatchGather {
   const SplitJob *jobs[kSplitGroups];
   const int *start[2 * kSplitGroups];
+  const int *counts;  // if not NULL: the groups' counts (element_tiled_batch), read instead of the two below
   int numJobs[kSplitGroups];
   int lines[2 * kSplitGroups];
 };
@@ -2385,18 +2388,20 @@ struct BatchGather {
 __global__ __launch_bounds__(256) void gather_batch(const BatchGather b) {
   const int64_t wave = uniform(int(blockIdx.x * 4 + threadIdx.x / 64)), waves = int64_t(gridDim.x) * 4;
   const int row = int(threadIdx.x % 64) / 4, h = int(threadIdx.x % 4);
+  auto lines = [&](int seg) { return b.counts ? cmem(b.counts)[4 * (seg / 2) + 2 + seg % 2] : b.lines[seg]; };
   int64_t steps = 0;
 #pragma unroll
-  for (int seg = 0; seg < 2 * kSplitGroups; seg++) steps += (b.lines[seg] + 15) / 16;
+  for (int seg = 0; seg < 2 * kSplitGroups; seg++) steps += (lines(seg) + 15) / 16;
   int64_t first = steps * wave / waves, last = steps * (wave + 1) / waves;  // of the steps that are left
 #pragma unroll 1
   for (int seg = 0; seg < 2 * kSplitGroups && last > 0; seg++) {
-    const int64_t here = (b.lines[seg] + 15) / 16;
+    const int64_t here = (lines(seg) + 15) / 16;
     if (first < here) {
-      const int end = int(min(16 * last, int64_t(b.lines[seg])));
+      const int end = int(min(16 * last, int64_t(lines(seg))));
       int at = int(16 * max(first, int64_t(0)));
       const int *start = b.start[seg];
-      for (int j = uniform(find_job(start, b.numJobs[seg / 2], at)); at < end; j++) {
+      const int numJobs = b.counts ? cmem(b.counts)[4 * (seg / 2)] : b.numJobs[seg / 2];
+      for (int j = uniform(find_job(start, numJobs, at)); at < end; j++) {
         const SplitJob job = b.jobs[seg / 2][j];
         const int j0 = start[j], jend = min(start[j + 1], end);
         for (; at < jend; at += 16) {
@@ -2450,6 +2455,39 @@ void launch_element_nl_order(int order, const ElemArgs &a, hipStream_t stream) {
   }
 }
 
+// Where a launch goes: a stream, or the end of a graph under construction, a chain of kernel nodes. (The nodes are added
+// by hand: while a stream is being captured, other threads' work on the default stream can fail.)
+struct GraphChain {
+  hipGraph_t graph = nullptr;
+  hipGraphNode_t last = nullptr;
+  hipError_t error = hipSuccess;  // of the first node that could not be added
+};
+struct Target {
+  hipStream_t stream;
+  GraphChain *chain = nullptr;
+  Target(hipStream_t s) : stream(s) {}
+  Target(GraphChain &c) : stream(nullptr), chain(&c) {}
+};
+
+template <typename... P>
+void launch(const Target &to, void (*kernel)(P...), unsigned grid, unsigned block, P... args) {
+  if (!to.chain) {
+    kernel<<<grid, block, 0, to.stream>>>(args...);
+    return;
+  }
+  GraphChain &c = *to.chain;
+  if (c.error != hipSuccess) return;
+  void *argv[] = {const_cast<void *>(static_cast<const void *>(&args))...};
+  hipKernelNodeParams node{};
+  node.func = reinterpret_cast<void *>(kernel);
+  node.gridDim = dim3(grid);
+  node.blockDim = dim3(block);
+  node.kernelParams = argv;
+  hipGraphNode_t added = nullptr;
+  c.error = hipGraphAddKernelNode(&added, c.graph, c.last ? &c.last : nullptr, c.last ? 1 : 0, &node);
+  c.last = added;
+}
+
 // One launch group: jobs of one order with the same outputs.
 struct OwnerLaunch {
   OwnerArgs args;
@@ -2463,7 +2501,7 @@ struct OwnerLaunch {
 };
 
 template <int P, typename T, int MAXR, bool RES, bool JAC, bool DET>
-void launch_owner(const OwnerLaunch &L, hipStream_t stream) {
+void launch_owner(const OwnerLaunch &L, const Target &to) {
   constexpr OwnerConfig cfg = owner_config(P);
   if constexpr (!DET && MAXR <= cfg.waves * 64) {
     if (L.stream) {
@@ -2472,55 +2510,55 @@ void launch_owner(const OwnerLaunch &L, hipStream_t stream) {
       const int grid = std::min(persistent, std::max((L.args.totalParts + 7) / 8, 1) * 8);
       auto *kernel = L.args.jobs ? owner_stream_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC, true>
                                  : owner_stream_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC, false>;
-      kernel<<<grid, cfg.waves * 64, 0, stream>>>(L.args);
+      launch(to, kernel, unsigned(grid), unsigned(cfg.waves * 64), L.args);
       return;
     }
   }
   const int grid = ((L.args.totalParts + 7) / 8) * 8;
-  owner_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC, DET><<<grid, cfg.waves * 64, 0, stream>>>(L.args);
+  owner_kernel<P, T, cfg.waves, cfg.maxBlocks, MAXR, RES, JAC, DET><<<grid, cfg.waves * 64, 0, to.stream>>>(L.args);
 }
 
 template <int P, typename T, bool DET>
-void launch_owner_mode(const OwnerLaunch &L, hipStream_t stream) {
+void launch_owner_mode(const OwnerLaunch &L, const Target &to) {
   constexpr OwnerConfig cfg = owner_config(P);
   if (L.jac && L.res) {
-    launch_owner<P, T, cfg.maxRows, true, true, DET>(L, stream);
+    launch_owner<P, T, cfg.maxRows, true, true, DET>(L, to);
   } else if (L.jac) {
-    launch_owner<P, T, cfg.maxRows, false, true, DET>(L, stream);
+    launch_owner<P, T, cfg.maxRows, false, true, DET>(L, to);
   } else if (L.rOnlyParts) {
     if constexpr (DET) {
-      launch_owner<P, T, kResidualOnlyMaxRows, true, false, true>(L, stream);
+      launch_owner<P, T, kResidualOnlyMaxRows, true, false, true>(L, to);
     } else {
       const int grid = (L.args.totalParts + 7) / 8 * 8;
       if (L.maxPartRows <= residual_rows(P)) {
-        residual_part_kernel<P, residual_rows(P)><<<grid, kLineWaves * 64, 0, stream>>>(L.args);
+        residual_part_kernel<P, residual_rows(P)><<<grid, kLineWaves * 64, 0, to.stream>>>(L.args);
       } else {
-        residual_part_kernel<P, kResidualOnlyMaxRows><<<grid, kLineWaves * 64, 0, stream>>>(L.args);
+        residual_part_kernel<P, kResidualOnlyMaxRows><<<grid, kLineWaves * 64, 0, to.stream>>>(L.args);
       }
     }
   } else {
     // Residual from a plan whose parts were sized for the Jacobian: rows fit the smaller bound.
-    launch_owner<P, T, cfg.maxRows, true, false, DET>(L, stream);
+    launch_owner<P, T, cfg.maxRows, true, false, DET>(L, to);
   }
 }
 
 template <int P>
-void launch_owner_order(const OwnerLaunch &L, hipStream_t stream) {
+void launch_owner_order(const OwnerLaunch &L, const Target &to) {
   if (L.precision == FEM_PREC_MIXED) {
-    if (L.det) launch_owner_mode<P, float, true>(L, stream);
-    else launch_owner_mode<P, float, false>(L, stream);
+    if (L.det) launch_owner_mode<P, float, true>(L, to);
+    else launch_owner_mode<P, float, false>(L, to);
   } else {
-    if (L.det) launch_owner_mode<P, double, true>(L, stream);
-    else launch_owner_mode<P, double, false>(L, stream);
+    if (L.det) launch_owner_mode<P, double, true>(L, to);
+    else launch_owner_mode<P, double, false>(L, to);
   }
 }
 
-void launch_owner_any(int order, const OwnerLaunch &L, hipStream_t stream) {
+void launch_owner_any(int order, const OwnerLaunch &L, const Target &to) {
   switch (order) {
-    case 1: launch_owner_order<1>(L, stream); break;
-    case 2: launch_owner_order<2>(L, stream); break;
-    case 3: launch_owner_order<3>(L, stream); break;
-    default: launch_owner_order<4>(L, stream); break;
+    case 1: launch_owner_order<1>(L, to); break;
+    case 2: launch_owner_order<2>(L, to); break;
+    case 3: launch_owner_order<3>(L, to); break;
+    default: launch_owner_order<4>(L, to); break;
   }
 }
 
@@ -3072,7 +3110,7 @@ struct fem_batch {
   };
   struct SplitGroup {
     std::vector<SplitJob> jobs;
-    std::vector<int> unitStart{0}, gStart{0}, rStart{0};  // prefix sums: units, staged blocks, staged residuals
+    std::vector<int> unitStart{0}, gStart{0}, rStart{0};  // prefix sums: units, block lines, residual lines
     std::vector<int64_t> stageOff, rstageOff;             // each job's staging, in doubles into the arena
   };
   static constexpr int kGroups = 12;
@@ -3086,9 +3124,9 @@ struct fem_batch {
   int flags = 0;
   int numCUs = 0;
   int numJobs = 0;
-  // One device block, laid out as
-  //   counts [kGroups + kSplitGroups][4] int (owner: numJobs, totalParts; element-once: numJobs, units,
-  //     staged blocks, staged residuals)
+  // One device block at a fixed address (recorded graphs refer to it), laid out as
+  //   counts [kGroups + kSplitGroups][4] int (owner: numJobs, totalParts; element-once: numJobs, units, block lines,
+  //     residual lines)
   //   | jobStart [kGroups][maxJobs + 1] int | jobs [kGroups][maxJobs] MeshJob
   //   | split starts [kSplitGroups][3][maxJobs + 1] int (unitStart, gStart, rStart)
   //   | split jobs [kSplitGroups][maxJobs] SplitJob
@@ -3108,6 +3146,16 @@ struct fem_batch {
   };
   std::vector<Solo> solo;
   bool assembled = false;  // fem_batch_assemble has staged job tables
+  bool current = false;    // the device's tables are the mirror's
+  // FEM_BATCH_GRAPH: recorded graphs by composition (see batch_graph); exec is NULL if recording failed.
+  using Composition = std::array<uint8_t, 1 + kGroups + kSplitGroups + 1>;
+  struct Recorded {
+    Composition key;
+    hipGraphExec_t exec;
+  };
+  static constexpr size_t kMaxRecorded = 64;
+  std::vector<Recorded> recorded;
+  bool prepared = false;  // batch_prepare has recorded what this batch replays; nothing is recorded later
 
   int *dCounts() const { return reinterpret_cast<int *>(dTables); }
   int *dJobStart() const { return reinterpret_cast<int *>(dTables + jobStartOffset); }
@@ -3115,7 +3163,7 @@ struct fem_batch {
   int *hCounts() const { return reinterpret_cast<int *>(hTables); }
   int *hJobStart() const { return reinterpret_cast<int *>(hTables + jobStartOffset); }
   MeshJob *hJobs() const { return reinterpret_cast<MeshJob *>(hTables + jobsOffset); }
-  // element-once group g: start array k (0 units, 1 staged blocks, 2 staged residuals) and jobs
+  // element-once group g: start array k (0 units, 1 block lines, 2 residual lines) and jobs
   size_t splitStartAt(int g, int k) const { return splitStartOffset + (size_t(g) * 3 + k) * (maxJobs + 1) * sizeof(int); }
   size_t splitJobsAt(int g) const { return splitJobsOffset + size_t(g) * maxJobs * sizeof(SplitJob); }
 };
@@ -3130,14 +3178,21 @@ void free_batch(fem_batch *b) {
   if (b->dArena) (void)hipFree(b->dArena);
   if (b->dTables) (void)hipFree(b->dTables);
   if (b->hTables) (void)hipHostFree(b->hTables);
+  // (freeing device memory has waited for the graphs' last replays)
+  for (auto &r : b->recorded) {
+    if (r.exec) (void)hipGraphExecDestroy(r.exec);
+  }
 }
 
-OwnerLaunch batch_group_launch(const fem_batch *b, int gi, int precision) {
+// Launch parameters of owner group gi. fromDevice: the kernel reads the group's counts from the device tables, and
+// numbers of parts here only size the grid.
+OwnerLaunch batch_group_launch(const fem_batch *b, int gi, int precision, bool fromDevice) {
   const fem_batch::Group &g = b->groups[gi];
   OwnerLaunch L{};
   make_basis(gi / 3 + 1, L.args.basis);
   L.args.jobs = b->dJobs() + size_t(gi) * b->maxJobs;
   L.args.jobStart = b->dJobStart() + size_t(gi) * (b->maxJobs + 1);
+  L.args.counts = fromDevice ? b->dCounts() + 4 * gi : nullptr;
   L.args.numJobs = int(g.jobs.size());
   L.args.totalParts = g.jobStart.back();
   L.precision = precision;
@@ -3145,52 +3200,132 @@ OwnerLaunch batch_group_launch(const fem_batch *b, int gi, int precision) {
   L.res = gi % 3 != 1;
   L.jac = gi % 3 != 0;
   L.rOnlyParts = false;
-  L.stream = g.stream && b->numCUs > 0;
+  L.stream = fromDevice || (g.stream && b->numCUs > 0);
   L.streamGrid = stream_grid(b->numCUs);
   return L;
 }
 
-// Launch of element-once group g (order 3 + g / 2; with residual if g is odd): the tiled kernel over the group's
-// units, whose counts it reads from device memory.
+// Most workgroups of a batch's element-once kernel and of its gather.
+int split_grid(const fem_batch *b) { return std::max(8 * b->numCUs, 64); }
+
+// Launch of element-once group g (order 3 + g / 2; with residual if g is odd): the tiled kernel over `units` units at
+// most, as many as the device's counts say.
 template <int P, typename T, bool RES>
-void launch_split_group_t(const fem_batch *b, int g, hipStream_t s) {
-  const fem_batch::SplitGroup &sg = b->split[g];
+void launch_split_group_t(const fem_batch *b, int g, int units, const Target &to) {
   const int *counts = b->dCounts() + 4 * (fem_batch::kGroups + g);
   const SplitJob *jobs = reinterpret_cast<const SplitJob *>(b->dTables + b->splitJobsAt(g));
   const int *unitStart = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 0));
-  const int cap = std::max(8 * b->numCUs, 64);
-  const unsigned grid = unsigned(std::clamp(sg.unitStart.back(), 1, cap));
+  const unsigned grid = unsigned(std::clamp(units, 1, split_grid(b)));
   Basis1D basis;
   make_basis(P, basis);
-  element_tiled_batch<P, T, kTiledWaves, RES><<<grid, kTiledWaves * 64, 0, s>>>(jobs, unitStart, counts, basis);
+  launch(to, &element_tiled_batch<P, T, kTiledWaves, RES>, grid, unsigned(kTiledWaves * 64), jobs, unitStart, counts, basis);
 }
 
-void launch_split_group(const fem_batch *b, int g, int precision, hipStream_t s) {
+void launch_split_group(const fem_batch *b, int g, int precision, int units, const Target &to) {
   const bool mixed = precision == FEM_PREC_MIXED;
   switch (g) {
-    case 0: mixed ? launch_split_group_t<3, float, false>(b, g, s) : launch_split_group_t<3, double, false>(b, g, s); break;
-    case 1: mixed ? launch_split_group_t<3, float, true>(b, g, s) : launch_split_group_t<3, double, true>(b, g, s); break;
-    case 2: mixed ? launch_split_group_t<4, float, false>(b, g, s) : launch_split_group_t<4, double, false>(b, g, s); break;
-    default: mixed ? launch_split_group_t<4, float, true>(b, g, s) : launch_split_group_t<4, double, true>(b, g, s); break;
+    case 0: mixed ? launch_split_group_t<3, float, false>(b, g, units, to) : launch_split_group_t<3, double, false>(b, g, units, to); break;
+    case 1: mixed ? launch_split_group_t<3, float, true>(b, g, units, to) : launch_split_group_t<3, double, true>(b, g, units, to); break;
+    case 2: mixed ? launch_split_group_t<4, float, false>(b, g, units, to) : launch_split_group_t<4, double, false>(b, g, units, to); break;
+    default: mixed ? launch_split_group_t<4, float, true>(b, g, units, to) : launch_split_group_t<4, double, true>(b, g, units, to); break;
   }
 }
 
-// Launch of the gathers of all element-once groups.
-void launch_split_gather(const fem_batch *b, hipStream_t s) {
-  BatchGather args{};
+// Workgroups that the gathers of all element-once groups take.
+int split_gather_blocks(const fem_batch *b) {
   int64_t lines = 0;
+  for (int g = 0; g < kSplitGroups; g++) lines += b->split[g].gStart.back() + (g % 2 ? int64_t(b->split[g].rStart.back()) : 0);
+  return int(std::clamp<int64_t>((4 * lines + 255) / 256, 1, split_grid(b)));
+}
+
+// Launch of those gathers, their counts read from the device tables or (fromDevice false) passed.
+void launch_split_gather(const fem_batch *b, bool fromDevice, int blocks, const Target &to) {
+  BatchGather args{};
+  args.counts = fromDevice ? b->dCounts() + 4 * fem_batch::kGroups : nullptr;
   for (int g = 0; g < kSplitGroups; g++) {
     const fem_batch::SplitGroup &sg = b->split[g];
     args.jobs[g] = reinterpret_cast<const SplitJob *>(b->dTables + b->splitJobsAt(g));
     args.numJobs[g] = int(sg.jobs.size());
-    for (int k = 0; k < 2; k++) {
-      args.start[2 * g + k] = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 1 + k));
-      if (k == 0 || g % 2 == 1) args.lines[2 * g + k] = (k ? sg.rStart : sg.gStart).back();
-      lines += args.lines[2 * g + k];
-    }
+    args.lines[2 * g] = sg.gStart.back();
+    args.lines[2 * g + 1] = g % 2 ? sg.rStart.back() : 0;
+    for (int k = 0; k < 2; k++) args.start[2 * g + k] = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 1 + k));
   }
-  const int cap = std::max(8 * b->numCUs, 64);
-  gather_batch<<<unsigned(std::clamp<int64_t>((4 * lines + 255) / 256, 1, cap)), 256, 0, s>>>(args);
+  launch(to, &gather_batch, unsigned(blocks), 256u, args);
+}
+
+// 0 for n = 0, else 1 + the exponent of the least power of two >= min(n, most); and that power.
+uint8_t size_class(int64_t n, int64_t most) {
+  uint8_t c = 0;
+  for (n = std::min(n, most); n > 0 && (int64_t(1) << c) < n; c++) {
+  }
+  return n > 0 ? uint8_t(c + 1) : 0;
+}
+int class_size(uint8_t c) { return 1 << (c - 1); }
+
+// Records a composition: precision, size class of every group's grid (0: not launched), of the gather's.
+void record_batch(fem_batch *b, const fem_batch::Composition &key) {
+  constexpr int G = fem_batch::kGroups, S = kSplitGroups;
+  const int precision = key[0];
+  GraphChain chain;
+  chain.error = hipGraphCreate(&chain.graph, 0);
+  for (int g = 0; g < G; g++) {
+    if (!key[1 + g]) continue;
+    OwnerLaunch L = batch_group_launch(b, g, precision, true);
+    L.args.totalParts = class_size(key[1 + g]);
+    launch_owner_any(g / 3 + 1, L, chain);
+  }
+  for (int g = 0; g < S; g++) {
+    if (key[1 + G + g]) launch_split_group(b, g, precision, class_size(key[1 + G + g]), chain);
+  }
+  if (key[1 + G + S]) launch_split_gather(b, true, class_size(key[1 + G + S]), chain);
+  hipGraphExec_t exec = nullptr;
+  if (chain.error == hipSuccess) chain.error = hipGraphInstantiate(&exec, chain.graph, nullptr, nullptr, 0);
+  if (chain.graph) (void)hipGraphDestroy(chain.graph);
+  if (chain.error != hipSuccess) {
+    (void)hipGetLastError();
+    exec = nullptr;
+  }
+  b->recorded.push_back({key, exec});
+}
+
+// The graph of a batch's launches, or NULL where they are to be issued directly. Graphs are kept by composition: the
+// precision, the groups that hold jobs and the sizes of their grids, rounded up to a power of two so that batches of
+// similar sizes share one. Everything else the kernels read from the job tables and counts in device memory, so a graph
+// serves whatever jobs the batch is refilled with.
+// A replay with unchanged tables (`changed` false) copies none and is faster than the launches; us a call, one after the
+// other, replayed and launched: 24 meshes of orders 1-4, mixed, 242 and 257; all twelve output groups 105 and 132; one
+// mesh of order 4 (36 elements, two launches) 22 and 38. Behind a copy of new tables the runtime starts a graph 6-8 us
+// later than a launch: 265, 138 and 45 us for the same three, so there only batches of at least kCopiedLaunches are
+// replayed, whose launches cost the host more (17 launches: 47 us, their replay 27). A single launch gains nothing.
+// Recorded when a batch is assembled again with unchanged tables (so the first assembly costs no recording; the second
+// 20-160 us more), up to kMaxRecorded; what is not recorded, also for want of memory, is launched directly.
+hipGraphExec_t batch_graph(fem_batch *b, int precision, bool changed) {
+  constexpr int G = fem_batch::kGroups, S = kSplitGroups, kCopiedLaunches = 8;
+  if (b->numCUs <= 0) return nullptr;
+  fem_batch::Composition key{};
+  key[0] = uint8_t(precision);
+  for (int g = 0; g < G; g++) key[1 + g] = size_class(b->groups[g].jobStart.back(), stream_grid(b->numCUs));
+  bool staged = false;
+  for (int g = 0; g < S; g++) {
+    key[1 + G + g] = size_class(b->split[g].unitStart.back(), split_grid(b));
+    staged = staged || key[1 + G + g] > 0;
+  }
+  if (staged) key[1 + G + S] = size_class(split_gather_blocks(b), split_grid(b));
+  const auto launches = std::count_if(key.begin() + 1, key.end(), [](uint8_t c) { return c != 0; });
+  if (launches < (changed ? kCopiedLaunches : 2)) return nullptr;
+  // A prepared graph, the one of small grids first, serves any batch of its groups that needs no larger ones.
+  auto covered = [](uint8_t need, uint8_t has) { return need <= has && (need == 0) == (has == 0); };
+  auto serves = [&](const fem_batch::Recorded &r) {
+    return r.key == key || (b->prepared && r.key[0] == key[0] &&
+                            std::equal(key.begin() + 1, key.end(), r.key.begin() + 1, covered));
+  };
+  auto it = std::find_if(b->recorded.begin(), b->recorded.end(), serves);
+  if (it == b->recorded.end()) {
+    if (changed || b->prepared || b->recorded.size() >= fem_batch::kMaxRecorded) return nullptr;
+    record_batch(b, key);
+    it = b->recorded.end() - 1;
+  }
+  return it->exec;
 }
 
 }  // namespace
@@ -3200,17 +3335,29 @@ int fem::batch_prepare(fem_batch *b, int precision) {
   if (precision != FEM_PREC_FP64 && precision != FEM_PREC_MIXED) {
     return set_error(FEM_ERR_INVALID_ARGUMENT, "unknown precision mode %d", precision);
   }
-  if (!(b->flags & FEM_BATCH_GRAPH) || b->assembled) return FEM_OK;  // until then the device tables are zero
+  if (!(b->flags & FEM_BATCH_GRAPH) || b->assembled || b->prepared) return FEM_OK;
   hipStream_t s = nullptr;
   FEM_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  for (int gi = 0; gi < fem_batch::kGroups; gi++) {
-    OwnerLaunch L = batch_group_launch(b, gi, precision);
-    L.stream = true;
-    launch_owner_any(gi / 3 + 1, L, s);
-  }
-  for (int g = 0; g < kSplitGroups; g++) launch_split_group(b, g, precision, s);
-  launch_split_gather(b, s);
+  // With the counts of the device tables, which are zero, also where jobs have been added but not assembled.
+  constexpr int G = fem_batch::kGroups, S = kSplitGroups;
+  for (int gi = 0; gi < G; gi++) launch_owner_any(gi / 3 + 1, batch_group_launch(b, gi, precision, true), s);
+  for (int g = 0; g < S; g++) launch_split_group(b, g, precision, 1, s);
+  launch_split_gather(b, true, 1, s);
   hipError_t e = hipGetLastError();
+  for (const int part : {16, 1}) {  // small grids and the largest
+    if (e != hipSuccess || b->numCUs <= 0) break;
+    const uint8_t owner = size_class(stream_grid(b->numCUs) / part, INT32_MAX), split = size_class(split_grid(b) / part, INT32_MAX);
+    fem_batch::Composition key{};
+    key[0] = uint8_t(precision);
+    for (int g = 0; g < G; g++) {  // residual alone at every order, and both outputs where the owner kernel forms them
+      if (g % 3 == 0 || (g % 3 == 2 && g < 6)) key[1 + g] = owner;
+    }
+    for (int g = 1; g < S; g += 2) key[1 + G + g] = split;
+    key[1 + G + S] = split;
+    record_batch(b, key);
+    b->prepared = true;
+    if (b->recorded.back().exec) e = hipGraphLaunch(b->recorded.back().exec, s);
+  }
   const hipError_t w = hipStreamSynchronize(s);
   (void)hipStreamDestroy(s);
   if (e == hipSuccess) e = w;
@@ -3407,41 +3554,55 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
   }
   // Counts of all groups and job tables of non-empty groups, staged in the mirror and copied up to the
   // end of the last non-empty group's jobs.
+  bool changed = false;
+  auto stage = [&](size_t at, const void *from, size_t bytes) {
+    if (std::memcmp(batch->hTables + at, from, bytes) == 0) return;
+    std::memcpy(batch->hTables + at, from, bytes);
+    changed = true;
+  };
   size_t copyEnd = batch->jobsOffset;
   for (int gi = 0; gi < fem_batch::kGroups; gi++) {
     fem_batch::Group &g = batch->groups[gi];
-    batch->hCounts()[4 * gi] = int(g.jobs.size());
-    batch->hCounts()[4 * gi + 1] = g.jobStart.back();
+    const int cnt[4] = {int(g.jobs.size()), g.jobStart.back(), 0, 0};
+    stage(4 * gi * sizeof(int), cnt, sizeof(cnt));
     if (g.jobs.empty()) continue;
-    std::memcpy(batch->hJobs() + size_t(gi) * batch->maxJobs, g.jobs.data(), g.jobs.size() * sizeof(MeshJob));
-    std::memcpy(batch->hJobStart() + size_t(gi) * (batch->maxJobs + 1), g.jobStart.data(),
-                g.jobStart.size() * sizeof(int));
-    copyEnd = batch->jobsOffset + (size_t(gi) * batch->maxJobs + g.jobs.size()) * sizeof(MeshJob);
+    const size_t jobsAt = batch->jobsOffset + size_t(gi) * batch->maxJobs * sizeof(MeshJob);
+    stage(jobsAt, g.jobs.data(), g.jobs.size() * sizeof(MeshJob));
+    stage(batch->jobStartOffset + size_t(gi) * (batch->maxJobs + 1) * sizeof(int), g.jobStart.data(),
+          g.jobStart.size() * sizeof(int));
+    copyEnd = jobsAt + g.jobs.size() * sizeof(MeshJob);
   }
   for (int g = 0; g < kSplitGroups; g++) {
     const fem_batch::SplitGroup &sg = batch->split[g];
-    int *cnt = batch->hCounts() + 4 * (fem_batch::kGroups + g);
-    cnt[0] = int(sg.jobs.size());
-    cnt[1] = sg.unitStart.back();
-    cnt[2] = sg.gStart.back();
-    cnt[3] = sg.rStart.back();
+    const int cnt[4] = {int(sg.jobs.size()), sg.unitStart.back(), sg.gStart.back(), g % 2 ? sg.rStart.back() : 0};
+    stage(4 * (fem_batch::kGroups + g) * sizeof(int), cnt, sizeof(cnt));
     if (sg.jobs.empty()) continue;
     const std::vector<int> *starts[3] = {&sg.unitStart, &sg.gStart, &sg.rStart};
-    for (int k = 0; k < 3; k++) {
-      std::memcpy(batch->hTables + batch->splitStartAt(g, k), starts[k]->data(), starts[k]->size() * sizeof(int));
-    }
-    std::memcpy(batch->hTables + batch->splitJobsAt(g), sg.jobs.data(), sg.jobs.size() * sizeof(SplitJob));
+    for (int k = 0; k < 3; k++) stage(batch->splitStartAt(g, k), starts[k]->data(), starts[k]->size() * sizeof(int));
+    stage(batch->splitJobsAt(g), sg.jobs.data(), sg.jobs.size() * sizeof(SplitJob));
     copyEnd = batch->splitJobsAt(g) + sg.jobs.size() * sizeof(SplitJob);
   }
-  FEM_HIP_CHECK(hipMemcpyAsync(batch->dTables, batch->hTables, copyEnd, hipMemcpyHostToDevice, s));
-  FEM_HIP_CHECK(hipEventRecord(batch->staged, s));
-  batch->stagedPending = true;
-  batch->assembled = true;
+  // A graph batch whose tables are those of its last assembly, whose copy has run, takes none.
+  changed = changed || !batch->current;
+  if (changed || !(batch->flags & FEM_BATCH_GRAPH)) {
+    batch->assembled = true;
+    batch->current = false;
+    FEM_HIP_CHECK(hipMemcpyAsync(batch->dTables, batch->hTables, copyEnd, hipMemcpyHostToDevice, s));
+    FEM_HIP_CHECK(hipEventRecord(batch->staged, s));
+    batch->stagedPending = true;
+    batch->current = true;
+  }
+  const hipGraphExec_t graph = (batch->flags & FEM_BATCH_GRAPH) ? batch_graph(batch, precision, changed) : nullptr;
   return timed(s, elapsedSeconds, [&]() -> int {
+    if (graph) {
+      const hipError_t e = hipGraphLaunch(graph, s);
+      if (e != hipSuccess) return set_error(FEM_ERR_HIP, "hipGraphLaunch failed: %s", hipGetErrorString(e));
+      return FEM_OK;
+    }
     for (int gi = 0; gi < fem_batch::kGroups; gi++) {
       fem_batch::Group &g = batch->groups[gi];
       if (g.jobs.empty()) continue;
-      const OwnerLaunch L = batch_group_launch(batch, gi, precision);
+      const OwnerLaunch L = batch_group_launch(batch, gi, precision, false);
       if (L.stream) {
         launch_owner_any(gi / 3 + 1, L, s);
       } else {
@@ -3459,10 +3620,10 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
     bool staged = false;
     for (int g = 0; g < kSplitGroups; g++) {
       if (batch->split[g].jobs.empty()) continue;
-      launch_split_group(batch, g, precision, s);
+      launch_split_group(batch, g, precision, batch->split[g].unitStart.back(), s);
       staged = true;
     }
-    if (staged) launch_split_gather(batch, s);
+    if (staged) launch_split_gather(batch, false, split_gather_blocks(batch), s);
     for (const fem_batch::Solo &j : batch->solo) {
       const int rc = fem::plan_assemble(j.plan, j.states, j.coords, j.E, j.nu, j.t, j.residual, j.values, precision, s,
                                         nullptr, false);

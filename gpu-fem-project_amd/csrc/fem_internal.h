@@ -129,9 +129,10 @@ int64_t batch_stage_doubles(const fem_plan *plan, bool withResidual);
 int batch_add_staged(fem_batch *batch, fem_plan *plan, const double *states, const double *nodeCoords, double E,
                      double nu, double t, double *residual, double *matEntries, double *stage);
 bool plan_streams_public(const fem_plan *plan);
-// Launches every group's kernels of a FEM_BATCH_GRAPH batch that was never assembled once, with no work, and waits, so
-// that the runtime's first-launch allocations (code, scratch of kernels that spill) happen now and not in the first
-// assembly. No-op without FEM_BATCH_GRAPH.
+// For a FEM_BATCH_GRAPH batch that was never assembled, the server's: launches every group's kernels once with no work,
+// records graphs of the server's full composition (residual-only and residual + Jacobian jobs of all orders; other
+// compositions are launched directly) and replays them with no work. The runtime's first-launch allocations (code,
+// scratch of kernels that spill, graph arguments) happen now, and none while serving. No-op without FEM_BATCH_GRAPH.
 int batch_prepare(fem_batch *batch, int precision);
 // fem_plan_assemble (accumulate false) and fem_plan_assemble_accumulate (true).
 int plan_assemble(fem_plan *plan, const double *states, const double *nodeCoords, double E, double nu, double t,

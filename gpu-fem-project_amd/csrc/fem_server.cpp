@@ -4,9 +4,10 @@
 // assembly requests (mesh, device states, residual-only or residual+Jacobian); the server allocates
 // each request's outputs when the request is admitted under the device-memory budget and keeps them
 // until the client releases them. A worker thread forms batches from the admitted requests and launches
-// each batch as fem_batch_assemble (one persistent launch per element order and output set) on one of several streams ("slots"): requests that arrive while
-// earlier batches run are collected into the next batch, which starts on a free slot and overlaps the
-// running ones on the device.
+// each batch as fem_batch_assemble (one persistent launch per element order and output set, where all are in use
+// optionally replayed through a recorded hipGraph) on one of several streams ("slots"): requests that arrive while
+// earlier batches run are collected into the next batch, which starts on a free slot and overlaps the running ones
+// on the device.
 //
 // Every device byte the server uses while serving comes from the budget: the resident meshes, and one arena
 // (sized at the first admission to what the budget leaves after them) holding each admitted request's outputs

@@ -287,9 +287,13 @@ int fem_plan_destroy(fem_plan *plan);
  * tables (asynchronously on `stream`) and launches; the batch may be cleared and refilled once the call
  * returns. */
 typedef struct fem_batch fem_batch;
-/* maxJobs: capacity per (order, outputs) group. flags: FEM_BATCH_GRAPH takes only jobs that run in the groups' own
- * launches, so that a call's launches do not grow with its jobs. (The launches of the groups that hold jobs are issued
- * directly: a recorded graph of all groups' launches is slower at every composition, also with all groups in use.) */
+/* maxJobs: capacity per (order, outputs) group. flags: FEM_BATCH_GRAPH records the launches of the groups that hold jobs
+ * as a hipGraph when the batch is assembled again with the same jobs (same plans, pointers and materials; the arrays'
+ * contents may differ) and replays it, without uploading the tables again. The graph's kernels read their counts and
+ * jobs from device memory, so it is kept for later contents of the batch with the same groups and similar sizes (up to
+ * 64 graphs). Behind new tables, where a graph starts later than a launch, only batches of many launches are replayed;
+ * the others are launched directly, as is a single launch. Such batches take only jobs that run in the groups'
+ * launches. */
 int fem_batch_create(int maxJobs, int flags, fem_batch **batch);
 #define FEM_BATCH_GRAPH 1
 int fem_batch_clear(fem_batch *batch);
@@ -314,7 +318,8 @@ typedef struct fem_server_config {
   int maxBatchJobs;       /* jobs per (order, outputs) group in one batch */
   int numSlots;           /* batches in flight (streams), 1..8 */
   int precision;          /* FEM_PREC_FP64 or FEM_PREC_MIXED */
-  int useGraphs;          /* batches are FEM_BATCH_GRAPH; their kernels are loaded when the server is created */
+  int useGraphs;          /* batches are FEM_BATCH_GRAPH: those that hold residual-only and residual + Jacobian jobs of
+                             all orders are replayed through graphs recorded when the server is created */
 } fem_server_config;
 
 int fem_server_create(const fem_server_config *cfg, fem_server **server);

@@ -10,7 +10,7 @@ namespace {
 std::mutex mu;
 std::map<void *, size_t> blocks;
 size_t used = 0, limit = size_t(1) << 40;
-int lastError = 0;
+int lastError = 0, launches = 0, graphLaunches = 0, graphNodes = 0, graphs = 0;
 struct Dim3 {
   unsigned x, y, z;
 };
@@ -20,6 +20,10 @@ extern "C" {
 
 void stub_limit(size_t bytes) { limit = bytes; }
 size_t stub_used() { return used; }
+int stub_launches() { return launches; }             // kernels launched directly
+int stub_graph_launches() { return graphLaunches; }  // graphs launched
+int stub_graph_nodes() { return graphNodes; }        // kernel nodes recorded
+int stub_graphs() { return graphs; }                 // executable graphs alive
 
 int hipMalloc(void **p, size_t n) {
   std::lock_guard<std::mutex> lk(mu);
@@ -63,7 +67,13 @@ int hipEventRecord(void *, void *) { return 0; }
 int hipEventSynchronize(void *) { return 0; }
 int hipEventQuery(void *) { return 0; }
 int hipEventElapsedTime(float *ms, void *, void *) { return *ms = 1, 0; }
-int hipLaunchKernel(const void *, Dim3, Dim3, void **, size_t, void *) { return 0; }
+int hipLaunchKernel(const void *, Dim3, Dim3, void **, size_t, void *) { return launches++, 0; }
+int hipGraphCreate(void **g, unsigned) { return *g = &mu, 0; }
+int hipGraphDestroy(void *) { return 0; }
+int hipGraphAddKernelNode(void **n, void *, void *const *, size_t, const void *) { return *n = &mu, graphNodes++, 0; }
+int hipGraphInstantiate(void **e, void *, void **, char *, size_t) { return *e = &mu, graphs++, 0; }
+int hipGraphLaunch(void *, void *) { return graphLaunches++, 0; }
+int hipGraphExecDestroy(void *) { return graphs--, 0; }
 int __hipPushCallConfiguration(Dim3, Dim3, size_t, void *) { return 0; }
 int __hipPopCallConfiguration(Dim3 *g, Dim3 *b, size_t *n, void **s) {
   *g = *b = Dim3{1, 1, 1};

@@ -60,6 +60,22 @@ void parallel_for(int64_t n, Fn fn, int64_t grain = 4096) {
   for (auto &th : pool) th.join();
 }
 
+// Sorts distinct keys: runs on all threads, then merges of neighbouring runs, half as many each time.
+void parallel_sort(std::vector<uint64_t> &keys) {
+  const int64_t n = int64_t(keys.size());
+  int64_t run = (n + hardware_threads() - 1) / hardware_threads();
+  run = std::max<int64_t>(run, 1 << 14);
+  auto at = [&](int64_t i) { return keys.begin() + std::min(n, i); };
+  parallel_for((n + run - 1) / run, [&](int64_t b, int64_t e) {
+    for (int64_t k = b; k < e; k++) std::sort(at(k * run), at((k + 1) * run));
+  }, 1);
+  for (; run < n; run *= 2) {
+    parallel_for((n + 2 * run - 1) / (2 * run), [&](int64_t b, int64_t e) {
+      for (int64_t k = 2 * b; k < 2 * e; k += 2) std::inplace_merge(at(k * run), at((k + 1) * run), at((k + 2) * run));
+    }, 1);
+  }
+}
+
 bool valid_order(int order) { return order >= 1 && order <= 4; }
 
 // 1-D knot positions of a structured axis: n elements on [0, 1], order p, cosine knots.
@@ -154,19 +170,18 @@ inline int find_sorted(const int *cols, int b, int e, int col) {
   return (p != cols + e && *p == col) ? int(p - cols) : -1;
 }
 
-// Distance of cell (x, y) of a 2^16 x 2^16 grid along the Hilbert curve.
+// Distance of cell (x, y) of a 2^16 x 2^16 grid along the Hilbert curve: from the coarsest bits down, the quadrant's
+// rank along the curve, then the cell's place within it in the quadrant's own frame (the lower quadrants are transposed,
+// the lower right one also turned by 180 degrees). Without branches, which no predictor gets right here.
 uint32_t hilbert2(uint32_t x, uint32_t y) {
   uint32_t d = 0;
-  for (uint32_t s = 1u << 15; s > 0; s >>= 1) {
-    const uint32_t rx = (x & s) != 0, ry = (y & s) != 0;
-    d += s * s * ((3 * rx) ^ ry);
-    if (!ry) {
-      if (rx) {
-        x = ~x;
-        y = ~y;
-      }
-      std::swap(x, y);
-    }
+  for (int bit = 15; bit >= 0; bit--) {
+    const uint32_t right = (x >> bit) & 1, lower = ((y >> bit) & 1) ^ 1;
+    d = 4 * d + ((3 * right) ^ lower ^ 1);
+    const uint32_t turn = 0u - (right & lower), transpose = 0u - lower;
+    const uint32_t swap = (x ^ y) & transpose;
+    x ^= swap ^ turn;
+    y ^= swap ^ turn;
   }
   return d;
 }
@@ -291,7 +306,7 @@ int build_plan_host(int order, int numNodes, int numElements, const int *connPtr
         key[size_t(n)] = (uint64_t(first) << 32) | uint32_t(n);
       }
     });
-    std::sort(key.begin(), key.end());
+    parallel_sort(key);
     for (int n = 0; n < numNodes; n++) order_nodes[n] = int(key[n] & 0xFFFFFFFFu);
   }
 

@@ -2380,15 +2380,16 @@ constexpr int kSplitGroups = 4;
 struct BatchGather {
   const SplitJob *jobs[kSplitGroups];
   const int *start[2 * kSplitGroups];
-  const int *counts;  // if not NULL: the groups' counts (element_tiled_batch), read instead of the two below
+  const int *counts;  // COUNTED: the groups' counts (element_tiled_batch), read instead of the two below
   int numJobs[kSplitGroups];
   int lines[2 * kSplitGroups];
 };
 
+template <bool COUNTED>
 __global__ __launch_bounds__(256) void gather_batch(const BatchGather b) {
   const int64_t wave = uniform(int(blockIdx.x * 4 + threadIdx.x / 64)), waves = int64_t(gridDim.x) * 4;
   const int row = int(threadIdx.x % 64) / 4, h = int(threadIdx.x % 4);
-  auto lines = [&](int seg) { return b.counts ? cmem(b.counts)[4 * (seg / 2) + 2 + seg % 2] : b.lines[seg]; };
+  auto lines = [&](int seg) { return COUNTED ? cmem(b.counts)[4 * (seg / 2) + 2 + seg % 2] : b.lines[seg]; };
   int64_t steps = 0;
 #pragma unroll
   for (int seg = 0; seg < 2 * kSplitGroups; seg++) steps += (lines(seg) + 15) / 16;
@@ -2400,7 +2401,7 @@ __global__ __launch_bounds__(256) void gather_batch(const BatchGather b) {
       const int end = int(min(16 * last, int64_t(lines(seg))));
       int at = int(16 * max(first, int64_t(0)));
       const int *start = b.start[seg];
-      const int numJobs = b.counts ? cmem(b.counts)[4 * (seg / 2)] : b.numJobs[seg / 2];
+      const int numJobs = COUNTED ? cmem(b.counts)[4 * (seg / 2)] : b.numJobs[seg / 2];
       for (int j = uniform(find_job(start, numJobs, at)); at < end; j++) {
         const SplitJob job = b.jobs[seg / 2][j];
         const int j0 = start[j], jend = min(start[j + 1], end);
@@ -3250,7 +3251,7 @@ void launch_split_gather(const fem_batch *b, bool fromDevice, int blocks, const 
     args.lines[2 * g + 1] = g % 2 ? sg.rStart.back() : 0;
     for (int k = 0; k < 2; k++) args.start[2 * g + k] = reinterpret_cast<const int *>(b->dTables + b->splitStartAt(g, 1 + k));
   }
-  launch(to, &gather_batch, unsigned(blocks), 256u, args);
+  launch(to, fromDevice ? &gather_batch<true> : &gather_batch<false>, unsigned(blocks), 256u, args);
 }
 
 // 0 for n = 0, else 1 + the exponent of the least power of two >= min(n, most); and that power.

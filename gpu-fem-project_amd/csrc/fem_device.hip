@@ -435,8 +435,8 @@ struct ElemArgs {
 // their nodes (equal ones by index), the order of the blocks in a BSR row. Any order adds the same. The adds are
 // bound by the 64-byte requests that the L2 takes (21 G/s, however much of a request is used), and an instruction
 // covers 16 blocks: in this order a row of 25 columns falls into fewer lines per instruction however its element's
-// nodes are numbered (order 4, 30 625 elements, corners numbered first, then edges, then interiors: 644 -> 606 us, 1.51
-// blocks a request; rows of one instruction and ascending numberings are unchanged).
+// nodes are numbered (order 4, 30 625 elements, corners numbered first, then edges, then interiors: the kernel alone
+// 644 -> 606 us, 1.51 blocks a request; rows of one instruction and ascending numberings are unchanged).
 // The nodes pass through `ids`, one slot per lane of the wavefront, free on return.
 template <int P>
 __device__ __forceinline__ int emission_slot(int *ids, int lane, int el, int idx, int node, bool valid) {
@@ -1465,8 +1465,8 @@ template <int P, typename T, bool JAC, bool ALL_LANES, typename Where, typename 
 __device__ __forceinline__ void stage_stiffness_rows(WaveLDS<P, T> &W, const double2 *gref, const Material &m, int el,
                                                      int b, bool valid, int count, int maxCount, double &Rx,
                                                      double &Ry, Where &&where, Emit &&emit) {
-  // FP64 chunks are halved to stay within 256 registers; 5 rows divide order 4's 25 (30 625 elements through atomics: 693
-  // us with 4 rows, 684 with 5, 688 with 8; owner-only plan of the annulus 60 x 300: 466 against 439), at order 3 4 rows
+  // FP64 chunks are halved to stay within 256 registers; 5 rows divide order 4's 25 (30 625 elements through atomics, with
+  // the zeroing of the outputs: 693 us with 4 rows, 684 with 5, 688 with 8; owner-only plan of the annulus 60 x 300: 466 against 439), at order 3 4 rows
   // are better than 8 (516 against 521 us).
   constexpr int CH = sizeof(T) == 8 ? (P == 4 ? 5 : 4) : 8;
   Rx = 0;
@@ -2422,8 +2422,8 @@ __global__ __launch_bounds__(256) void gather_batch(const BatchGather b) {
   }
 }
 
-// Element-once assembly of one plan: the element kernel stores exclusive outputs and stages the rest, then
-// the gathers store the staged sums.
+// Element-once assembly of one plan: the element kernel stores the first contribution to each output and stages the
+// others, then the gathers add them (GatherList).
 template <int P>
 void launch_split(const SplitJob &job, const Basis1D &basis, int precision, int waves, hipStream_t s) {
   const bool res = job.residual != nullptr;
@@ -2860,8 +2860,8 @@ int create_plan(int order, int numNodes, int numElements, const int *connPtr, co
     return rc;
   }
   // Orders 3-4: Jacobian assemblies traverse the elements once (the owner-computes parts visit each element
-  // 3-4 times there). Most blocks of an element's K_e are formed by that element alone and are stored
-  // directly; the rest are staged and summed by a gather pass (SplitHost). Without room for int codes the
+  // 3-4 times there). Most blocks of an element's K_e are formed by that element alone or first and are stored
+  // directly; the rest are staged and added by a gather pass (GatherList). Without room for int codes the
   // plan keeps the owner-computes path (as FEM_PLAN_OWNER_ONLY plans do).
   if (order >= 3 && !(flags & (FEM_PLAN_RESIDUAL_ONLY | FEM_PLAN_OWNER_ONLY))) {
     const int N = (order + 1) * (order + 1);
@@ -3072,7 +3072,7 @@ int fem::plan_assemble(fem_plan *plan, const double *states, const double *nodeC
   L.stream = plan_streams(plan);
   L.streamGrid = stream_grid(plan->numCUs);
   if (plan->dConn && matEntries) {
-    // Element-once assembly (orders 3-4): exclusive outputs stored by their element, the rest staged and
+    // Element-once assembly (orders 3-4): first contributions stored by their element, the others staged and
     // gathered. Deterministic, so it also serves FEM_PLAN_DETERMINISTIC plans.
     SplitJob job = make_split_job(plan, states, nodeCoords, residual, matEntries, m);
     job.accumulate = accumulate ? 1 : 0;

@@ -30,8 +30,8 @@ struct OwnerConfig {
 };
 // Orders 1-2: one workgroup of 8 waves per CU (two per SIMD) sharing an accumulator of 2720 FP64 blocks,
 // so parts are twice as large as with two 4-wave workgroups and fewer elements are visited twice
-// (1.53 visits per element at 1000x1000 order 2, against 1.83). Orders 3-4: two workgroups of 4 waves
-// per CU, each with half the LDS.
+// (1.45 visits per element at 1000x1000 order 2; along a Morton curve 1.53, against 1.83 for the smaller parts).
+// Orders 3-4: two workgroups of 4 waves per CU, each with half the LDS.
 constexpr OwnerConfig owner_config(int order) {
   return order == 1   ? OwnerConfig{8, 2720, 352, 128}
          : order == 2 ? OwnerConfig{8, 2720, 320, 56}
@@ -75,11 +75,9 @@ struct PlanHost {
 };
 
 // Element-once tables (orders 3-4). Every output (a BSR block, or a node's residual pair) is either
-// exclusive, formed by exactly one (element, node[, node]) contribution, or not. An exclusive output is
-// stored by its one contributor; the contributions to any other output go to slots of a staging array,
-// grouped by output, and a gather pass stores each such output as the sum of its slots in slot order (zero
-// when no element touches it). Every output is written exactly once and the result is bitwise
-// reproducible.
+// exclusive, formed by exactly one (element, node[, node]) contribution, or not. The contributions to any other
+// output have slots, grouped by output, and the output is the sum of its slots in slot order (zero when no element
+// touches it), so the result is bitwise reproducible. Plans keep these tables in the form of GatherList.
 struct SplitHost {
   std::vector<int> code;   // [E][N][N], row-major (a, b): block of rows conn[e,a] x column conn[e,b]; below
                            // numBlocks the block's BSR index (exclusive), else numBlocks + staging slot

@@ -10,7 +10,8 @@
 //      ids -> row lengths -> exclusive scan -> rowp. Rows of more elements go to a list that wavefronts work
 //      through: they sort the row's node references in LDS (bitonic network);
 //   3. the same again writes the distinct ids into cols;
-//   4. the map: one thread per (element, i, j), binary search of node j in row i.
+//   4. the map: a workgroup copies the rows of a few elements to LDS and searches each (element, i, j) there
+//      (elements of 4, 9, 16 or 25 nodes; else one thread per entry searches row i in global memory).
 // Invalid node ids, rows with more candidates than a wavefront sorts, and map misses raise device flags
 // that the host turns into status codes; no access depends on an unchecked id.
 

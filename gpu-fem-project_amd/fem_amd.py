@@ -452,7 +452,8 @@ def bsr_spmv(pattern_rowp, pattern_cols, values, x, y, stream=None):
 
 
 class Plan:
-    """Resident owner-computes assembly plan (fem_plan_*)."""
+    """Resident assembly plan (fem_plan_*). morton: give the plan the mesh's coordinates, along whose space-filling
+    curve its parts are cut (else in the nodes' own order)."""
 
     def __init__(self, mesh: Mesh, pattern: Pattern, flags: int = 0, morton: bool = True):
         self._lib = load()

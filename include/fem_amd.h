@@ -223,17 +223,18 @@ int fem_jacobian_coloured(int order, const int *connPtr, const int *conn, int nu
                           const int *colourElements, const int *colourPtr, int numColours, double *residual,
                           double *matEntries, int precision, void *stream, double *elapsedSeconds);
 
-/* ---- resident assembly plan (owner-computes, write-once) ---------------------------------------
+/* ---- resident assembly plan (no zero-fill, no atomics to HBM) ----------------------------------
  * Built once per mesh from host arrays, kept on the device. Nodes are split into parts whose BSR
  * rows fit a workgroup's LDS; each workgroup assembles every element touching its rows and writes
  * its residual entries and BSR blocks exactly once (no atomics to HBM, no zero-fill). Results are
  * written (not accumulated) into the caller's residual / values in the layout of `rowp`/`cols`.
  * nodeCoordsHost (optional) orders nodes along a Hilbert curve through the elements, so parts are compact.
- * At orders 3-4 a plan also holds element-once tables: a Jacobian assembly visits each element once,
- * stores the blocks (and residual entries) that element alone forms, stages the others in the plan's
- * staging buffer and sums them in a gather pass; every output is still written exactly once, in a fixed
- * order, so results are bitwise reproducible with or without FEM_PLAN_DETERMINISTIC. A plan's job record
- * and staging buffer are per plan: assemblies of one plan must not overlap on different streams. */
+ * At orders 3-4 a plan also holds element-once tables: a Jacobian assembly visits each element once and stores
+ * the first contribution to each block (and residual entry) in place; further contributions go to the plan's
+ * staging buffer, and a gather pass reads each 64-byte line of the outputs that has some, adds them and stores
+ * the line again. The order of the sums is fixed, so results are bitwise reproducible with or without
+ * FEM_PLAN_DETERMINISTIC. The staging buffer is the plan's own: Jacobian assemblies of one plan of orders 3-4
+ * must not overlap on different streams. */
 typedef struct fem_plan fem_plan;
 
 int fem_plan_create(int order, int numNodes, int numElements, const int *connPtr, const int *conn,
@@ -267,7 +268,8 @@ int fem_plan_info(const fem_plan *plan, int64_t *numParts, int64_t *numBlocks, i
 int fem_plan_assemble(fem_plan *plan, const double *states, const double *nodeCoords, double E, double nu, double t,
                       double *residual, double *matEntries, int precision, void *stream, double *elapsedSeconds);
 /* fem_plan_assemble that adds its sums to residual / matEntries (+=, the reference kernels' semantics) instead of
- * storing them: each output is still read and written once (element-once plans still write their own staging). */
+ * storing them. Owner-computes plans read and write each output once; element-once plans add the first contribution
+ * to an output in place and the staged ones in the gather pass. */
 int fem_plan_assemble_accumulate(fem_plan *plan, const double *states, const double *nodeCoords, double E, double nu,
                                  double t, double *residual, double *matEntries, int precision, void *stream,
                                  double *elapsedSeconds);

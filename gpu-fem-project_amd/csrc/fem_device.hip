@@ -3583,17 +3583,22 @@ int fem_batch_assemble(fem_batch *batch, int precision, void *stream, double *el
     stage(batch->splitJobsAt(g), sg.jobs.data(), sg.jobs.size() * sizeof(SplitJob));
     copyEnd = batch->splitJobsAt(g) + sg.jobs.size() * sizeof(SplitJob);
   }
-  // A graph batch whose tables are those of its last assembly, whose copy has run, takes none.
+  // A graph batch whose tables are those of its last assembly, whose copy has run, takes none. In a capture of the
+  // caller's the copy and the launches themselves are recorded.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const bool graphs = (batch->flags & FEM_BATCH_GRAPH) != 0;
+  if (graphs && hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+  const bool replay = graphs && capture == hipStreamCaptureStatusNone;
   changed = changed || !batch->current;
-  if (changed || !(batch->flags & FEM_BATCH_GRAPH)) {
+  if (changed || !replay) {
     batch->assembled = true;
     batch->current = false;
     FEM_HIP_CHECK(hipMemcpyAsync(batch->dTables, batch->hTables, copyEnd, hipMemcpyHostToDevice, s));
     FEM_HIP_CHECK(hipEventRecord(batch->staged, s));
     batch->stagedPending = true;
-    batch->current = true;
+    batch->current = replay;  // (a captured copy has not run)
   }
-  const hipGraphExec_t graph = (batch->flags & FEM_BATCH_GRAPH) ? batch_graph(batch, precision, changed) : nullptr;
+  const hipGraphExec_t graph = replay ? batch_graph(batch, precision, changed) : nullptr;
   return timed(s, elapsedSeconds, [&]() -> int {
     if (graph) {
       const hipError_t e = hipGraphLaunch(graph, s);

@@ -60,6 +60,7 @@ int hipDeviceSynchronize() { return 0; }
 int hipStreamCreateWithFlags(void **s, unsigned) { return *s = &mu, 0; }
 int hipStreamDestroy(void *) { return 0; }
 int hipStreamSynchronize(void *) { return 0; }
+int hipStreamIsCapturing(void *, int *status) { return *status = 0, 0; }
 int hipEventCreate(void **e) { return *e = &mu, 0; }
 int hipEventCreateWithFlags(void **e, unsigned) { return *e = &mu, 0; }
 int hipEventDestroy(void *) { return 0; }

@@ -129,3 +129,29 @@ def test_prepare_with_jobs(fem, torch_gpu, cases):
     batch.close()
     for p in plans:
         p.close()
+
+
+@pytest.mark.parametrize("warm", [0, 3])
+def test_in_a_capture(fem, torch_gpu, cases, warm):
+    """A batch of orders 1-2 assembled under the caller's own capture, before any other assembly or after replays:
+    the caller's graph uploads the tables and launches the kernels itself."""
+    torch = torch_gpu
+    which = [(0, True, True), (1, True, True), (1, True, False)]
+    plans = [fem.Plan(c["mesh"], c["pat"]) for c in cases]
+    batch = fem.Batch(max_jobs=4, graph=True)
+    filled = Filled(torch, batch, cases, plans, which, 1.0)
+    stream = torch.cuda.Stream()
+    for _ in range(warm):
+        batch.assemble(stream=stream)
+        filled.check(0)
+    graph = torch.cuda.CUDAGraph()
+    print(f"captured batch: warm {warm}", flush=True)
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        batch.assemble(stream=stream)
+    for _ in range(3):
+        graph.replay()
+        filled.check(0)
+    del graph
+    batch.close()
+    for p in plans:
+        p.close()
